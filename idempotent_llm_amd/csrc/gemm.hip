@@ -490,32 +490,48 @@ __global__ __launch_bounds__(64 * NW) void k_gemv_static(GemvArgs g, const int64
   }
 }
 
-// Skinny GEMM over many columns (the LM head) for M <= 16 rows: the A rows
+// Skinny GEMM over many columns (the LM head): the A rows (MB groups of 16)
 // are staged in LDS once per block, and each wave walks its own 16-column
 // groups over the whole K range (grid-stride), with all of a group's weight
 // loads (up to 1024 bytes of K per lane) in flight before its MFMAs; no
-// cross-wave reduction. At the LM-head shape (N = 151936, K = 1024) it
-// streams 5.9 TB/s at M = 8 against 4.8 TB/s for the K-split tile.
+// cross-wave reduction, and every weight is read once whatever MB is. At the
+// LM-head shape (N = 151936, K = 1024, 155 MB of weights) the stream bounds
+// it: 33 us at M = 1, 36.5 at 16, 40.4 at 32 and 48.1 at 64 (the int32
+// product adds 10 to 39 MB). Above 16 rows it replaces the K-split tile of
+// k_gemv_nt, whose blocks each hold one 16-column group in flight: 76.2 us
+// at 32 rows, 121 at 64.
+// A row in LDS takes K + GS_PAD bytes: 16 rows K = 1024 apart would start in
+// the same bank.
 constexpr int GS_BLOCKS = 512;
-constexpr int GS_KMAX = 4096;  // A in LDS: 16 rows x K bytes
+constexpr int GS_KMAX = 4096;
+constexpr int GS_PAD = 16;
+constexpr int GS_LDS = 80 * 1024;  // two blocks per CU: 64 rows to K = 1024, 16 to 4096
 
+__host__ __device__ inline int gs_lds_bytes(int mb, int K) { return mb * 16 * (K + GS_PAD); }
+
+template <int MB>
 __global__ __launch_bounds__(256) void k_gemv_stream(const int8_t* __restrict__ A,
                                                      const int8_t* __restrict__ B,
                                                      int32_t* __restrict__ C, int M, int N,
                                                      int K, Prefetch pf) {
   keep_hidden_args();
-  extern __shared__ __attribute__((aligned(16))) int8_t sa[];  // [16][K]
+  extern __shared__ __attribute__((aligned(16))) int8_t sa[];  // [16 MB][K + GS_PAD]
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const PrefetchHold ph = prefetch_issue(pf, (i64)blockIdx.x * 256 + tid);
-  for (int i = tid * 16; i < 16 * K; i += 256 * 16)
-    *(v4i*)(sa + i) = i / K < M ? *(const v4i*)(A + i) : zero4();
+  const int ld = K + GS_PAD, kc = K >> 4;
+  for (int i = tid; i < 16 * MB * kc; i += 256) {
+    const int row = i / kc, k = (i - row * kc) * 16;
+    *(v4i*)(sa + row * ld + k) = row < M ? *(const v4i*)(A + (i64)row * K + k) : zero4();
+  }
   __syncthreads();
   const int r16 = lane & 15, grp = lane >> 4;
   const int groups = (N + 15) / 16;
   for (int gidx = blockIdx.x * 4 + wave; gidx < groups; gidx += gridDim.x * 4) {
     const int col = gidx * 16 + r16;
     const int8_t* brow = B + (i64)(col < N ? col : N - 1) * K;
-    v4i acc = zero4();
+    v4i acc[MB];
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) acc[mb] = zero4();
     for (int k0 = 0; k0 < K; k0 += 1024) {
       // lane (r16, grp) takes bytes grp * 16 .. + 15 of every 64-byte K slice
       // of column r16 and of A row r16 (the same K order on both operands)
@@ -528,15 +544,20 @@ __global__ __launch_bounds__(256) void k_gemv_stream(const int8_t* __restrict__ 
 #pragma unroll
       for (int u = 0; u < 16; ++u) {
         const int kk = k0 + u * 64 + grp * 16;
-        const v4i a = kk < K ? *(const v4i*)(sa + r16 * K + kk) : zero4();
-        acc = mfma16(a, b[u], acc);
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb) {
+          const v4i a = kk < K ? *(const v4i*)(sa + (mb * 16 + r16) * ld + kk) : zero4();
+          acc[mb] = mfma16(a, b[u], acc[mb]);
+        }
       }
     }
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int row = grp * 4 + r;
-      if (row < M && col < N) C[(i64)row * N + col] = acc[r];
-    }
+    for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int row = mb * 16 + grp * 4 + r;
+        if (row < M && col < N) C[(i64)row * N + col] = acc[mb][r];
+      }
   }
   prefetch_keep(pf, ph);
 }
@@ -669,8 +690,8 @@ void launch_gemv(dim3 grid, hipStream_t s, const int8_t* A, const int8_t* B, int
 // Skinny GEMM for M <= 64: writes ksplit int32 partials C[ks][M][N]
 // (split_stride elements apart); ksplit = 1 gives the plain product. Four
 // waves share one 16-column group and split its K range (measured faster than
-// a column group per wave at every layer shape); the LM head (N >= 32768,
-// M <= 16, no split) takes k_gemv_stream instead.
+// a column group per wave at every layer shape); the LM head (N >= 32768, no
+// split, A rows within GS_LDS) takes k_gemv_stream instead.
 int igemv(const int8_t* A, const int8_t* B, int32_t* C, int M, int N, int K, int ksplit,
           int64_t split_stride, const Prefetch& pf, hipStream_t s) {
   if (M <= 0 || N <= 0) return DI_OK;
@@ -680,11 +701,20 @@ int igemv(const int8_t* A, const int8_t* B, int32_t* C, int M, int N, int K, int
   const int kchunk = gemv_kchunk(K, ksplit);
   const int nsp = (K + kchunk - 1) / kchunk;
   if (nsp != ksplit) return DI_EINVAL;  // caller must size partial buffers to ksplit
-  if (ksplit == 1 && M <= 16 && N >= 32768 && K <= GS_KMAX) {
+  const int mb = (M + 15) / 16;
+  if (ksplit == 1 && N >= 32768 && K <= GS_KMAX && gs_lds_bytes(mb, K) <= GS_LDS) {
     const int groups = (N + 15) / 16;
     const int blocks = (groups + 3) / 4 < GS_BLOCKS ? (groups + 3) / 4 : GS_BLOCKS;
-    hipLaunchKernelGGL(k_gemv_stream, dim3(blocks), dim3(256), (size_t)16 * K, s, A, B, C, M, N,
-                       K, pf);
+    const size_t lds = (size_t)gs_lds_bytes(mb, K);
+#define DI_GS_LAUNCH(MB)                                                                        \
+  hipLaunchKernelGGL(k_gemv_stream<MB>, dim3(blocks), dim3(256), lds, s, A, B, C, M, N, K, pf)
+    switch (mb) {
+      case 1: DI_GS_LAUNCH(1); break;
+      case 2: DI_GS_LAUNCH(2); break;
+      case 3: DI_GS_LAUNCH(3); break;
+      default: DI_GS_LAUNCH(4); break;
+    }
+#undef DI_GS_LAUNCH
     DI_LAUNCH_CHECK();
     return DI_OK;
   }
@@ -696,7 +726,7 @@ int igemv(const int8_t* A, const int8_t* B, int32_t* C, int M, int N, int K, int
     DI_LAUNCH_CHECK();
     return DI_OK;
   }
-  switch ((M + 15) / 16) {
+  switch (mb) {
     case 1: launch_gemv<1, 4, 2>(grid, s, A, B, C, M, N, K, kchunk, ss, pf); break;
     case 2: launch_gemv<2, 4, 2>(grid, s, A, B, C, M, N, K, kchunk, ss, pf); break;
     case 3: launch_gemv<3, 4, 1>(grid, s, A, B, C, M, N, K, kchunk, ss, pf); break;
