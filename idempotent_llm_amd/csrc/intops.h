@@ -506,6 +506,25 @@ DI_HD int32_t rhad_est_corr_signed(i64 a, int s, i64 d, const DivEst& D) {
   return a < 0 ? -(int32_t)q : (int32_t)q;
 }
 
+// clamp_i8(rhad(n, d)) for |n| < 2^62 and 1 <= d < 2^52, D = make_divest of
+// an s = 1 divisor: e = fma(fl(|n|), D.r, D.k) is (|n| + floor(d/2) + 1/2) / d
+// within 2^-42 wherever that is below 256 (relative 2^-53 on |n|, D.r, D.k and
+// the fma), so its truncation is the quotient or one off it, and the exact
+// remainder settles it (the quotient is below 256, so |n| < 2^61 and q d <
+// 2^61). From e = 255 on the quotient is at least 254 and clamps.
+DI_HD int rhad_est_i8_corr(i64 n, i64 d, const DivEst& D) {
+  const i64 a = n < 0 ? -n : n;
+  const double e = fma((double)a, D.r, D.k);
+  i64 q = 255;
+  if (e < 255.0) {
+    q = (i64)(uint32_t)e;
+    const i64 rem = a + (d >> 1) - q * d;
+    q += (rem >= d ? 1 : 0) - (rem < 0 ? 1 : 0);
+  }
+  const int sq = n < 0 ? -(int)q : (int)q;
+  return sq < -128 ? -128 : (sq > 127 ? 127 : sq);
+}
+
 // sigmoid division round_half_away_div(num << 7, den) (ops/di_swiglu.py:
 // 52-55) for 0 <= num <= den < 2^31, den >= 1: the quotient v = (128 num +
 // floor(den/2)) / den is at most 128.5; fl((128 num + floor(den/2) + 1/2) /

@@ -140,6 +140,25 @@ struct HeadRed {
   }
 };
 
+// A mantissa operand of qk_head_f64 as an exact double, and whether it lies
+// inside the bound that needs (a float, which holds any integer below 2^24,
+// was checked when it was made: it takes half a double's registers).
+constexpr i64 QKV_WM_LIM = (i64)1 << 21, QKV_G_LIM = (i64)1 << 12, QKV_QS_LIM = (i64)1 << 15;
+__device__ __forceinline__ double mant_f64(i64 x) { return (double)(int32_t)x; }
+__device__ __forceinline__ double mant_f64(float x) { return (double)x; }
+__device__ __forceinline__ bool mant_ok(i64 x, i64 lim) { return in_range(x, lim); }
+__device__ __forceinline__ bool mant_ok(float, i64) { return true; }
+
+// requant_i8_static(kk, 1, k_rowk, 1, 0, kq_m, kq_k) of one rotated K value
+// (an exact double below 2^52): n = r << up, rhad(n, den) clamped
+__device__ __forceinline__ int kq_quant(double r, const KqChan& q) {
+  const double n = ldexp(r, (int)imin(q.up, 64));
+  const i64 lim = (i64)1 << 49;  // 2 |n| + den < 2^51 for the estimate
+  return (q.den > 0 && q.den < lim && fabs(n) < 0x1p49)
+             ? rhad_est_i8_f64(n, q.D)
+             : (int)clamp_i8(rhad(shl((i64)r, q.up), q.den));
+}
+
 // _qk_head_pipeline (model.py:200-216: requant_i32_common(16), di_rmsnorm,
 // gamma, apply_int_rope) then the K requantisation (model.py:326-329) or the
 // Q smoothing (model.py:317-320) and the Q quantiser's quotients
@@ -163,23 +182,26 @@ struct HeadRed {
 // Returns false (uniform over the head's lanes) for a head outside them, or
 // a zero head: the caller runs the integer routines. On true, o holds the K
 // head's int8 values or the Q head's quotients and *am_out the Q head's
-// max(max |q|, 1). kq(i): the KqChan of channel i (K heads only).
-template <int N, bool WAVE, class KqF>
+// max(max |q|, 1). W: int64 mantissas, checked here, or floats that the
+// caller checked (ok0) and made once for several rows.
+// kquant(r, o): the K head's int8 values from its rotated ones (false: it
+// could not, and the head takes the integer routines).
+template <int N, bool WAVE, class W, class KqF>
 __device__ __forceinline__ bool qk_head_f64(bool is_q, const int32_t (&p)[N],
-                                            const i64 (&wm)[N], const i64 (&gm)[N],
+                                            const W (&wm)[N], const W (&gm)[N],
                                             const int32_t (&cs)[N], const int32_t (&sn)[N],
-                                            const i64 (&qs)[N], KqF&& kq, int (&o)[N],
+                                            const W (&qs)[N], bool ok0, KqF&& kquant, int (&o)[N],
                                             i64* am_out) {
   constexpr int H = N / 2;
-  constexpr i64 WM_LIM = (i64)1 << 21, G_LIM = (i64)1 << 12, QS_LIM = (i64)1 << 15;
   const HeadRed<WAVE> red;
   double y[N];
   uint32_t pm = 0u;
-  bool ok = true;
+  bool ok = ok0;
 #pragma unroll
   for (int i = 0; i < N; ++i) {
-    ok = ok & in_range(wm[i], WM_LIM) & in_range(gm[i], G_LIM) & (!is_q | in_range(qs[i], QS_LIM));
-    y[i] = (double)p[i] * (double)(int32_t)wm[i];
+    ok = ok & mant_ok(wm[i], QKV_WM_LIM) & mant_ok(gm[i], QKV_G_LIM) &
+         (!is_q | mant_ok(qs[i], QKV_QS_LIM));
+    y[i] = (double)p[i] * mant_f64(wm[i]);
     pm = ::max(pm, f64_hiword_abs(y[i]));
   }
   const uint32_t L = bitlen_from_hiword(red.max_u32(ok ? pm : 0x7FF00000u));
@@ -205,7 +227,7 @@ __device__ __forceinline__ bool qk_head_f64(bool is_q, const int32_t (&p)[N],
   double a[N];
 #pragma unroll
   for (int i = 0; i < N; ++i)
-    a[i] = (double)rhad_est_signed_f64(y[i] * su, D) * (double)(int32_t)gm[i];
+    a[i] = (double)rhad_est_signed_f64(y[i] * su, D) * mant_f64(gm[i]);
   // apply_int_rope (rope.py:38-55)
   double r[N];
 #pragma unroll
@@ -214,24 +236,14 @@ __device__ __forceinline__ bool qk_head_f64(bool is_q, const int32_t (&p)[N],
     r[i + H] = rshift_round_f64(fma(a[i + H], (double)cs[i + H], a[i] * (double)sn[i + H]), 14);
   }
   if (!is_q) {
-    // requant_i8_static(kk, 1, k_rowk, 1, 0, kq_m, kq_k): n = r << up
-#pragma unroll
-    for (int i = 0; i < N; ++i) {
-      const KqChan q = kq(i);
-      const double n = ldexp(r[i], (int)imin(q.up, 64));
-      const i64 lim = (i64)1 << 49;  // 2 |n| + den < 2^51 for the estimate
-      o[i] = (q.den > 0 && q.den < lim && fabs(n) < 0x1p49)
-                 ? rhad_est_i8_f64(n, q.D)
-                 : (int)clamp_i8(rhad(shl((i64)r[i], q.up), q.den));
-    }
-    return true;
+    return kquant(r, o);
   }
   // QK smoothing, then quant_i8_pertoken's quotients (quant_row's two forms)
   double q[N];
   double g = 0.0;
 #pragma unroll
   for (int i = 0; i < N; ++i) {
-    q[i] = r[i] * (double)(int32_t)qs[i];
+    q[i] = r[i] * mant_f64(qs[i]);
     g = fmax(g, fabs(q[i]));
   }
   const double amu = f64_from_bits(red.max(f64_bits(g)));
@@ -496,7 +508,13 @@ __device__ __forceinline__ void qkv_head_compute(const QKVArgs& a, int r, int sl
     const int32_t pp[2] = {(int32_t)p0, (int32_t)p1}, cc[2] = {(int32_t)cs0, (int32_t)cs1},
                   ss[2] = {(int32_t)sn0, (int32_t)sn1};
     const i64 ww[2] = {wm0, wm1}, gg[2] = {g0, g1}, qq[2] = {qs0, qs1};
-    done = qk_head_f64<2, true>(is_q, pp, ww, gg, cc, ss, qq, kq, o, &am);
+    done = qk_head_f64<2, true>(is_q, pp, ww, gg, cc, ss, qq, true,
+                                [&](const double (&rv)[2], int (&ov)[2]) {
+#pragma unroll
+                                  for (int i = 0; i < 2; ++i) ov[i] = kq_quant(rv[i], kq(i));
+                                  return true;
+                                },
+                                o, &am);
   }
   if (DI_UNLIKELY(!done)) {
     // the integer routines (same integers, any operands)
@@ -583,48 +601,72 @@ __device__ __forceinline__ void qkv_head(const QKVArgs& a, int r, int slotw, int
 
 namespace di {
 
-// ---- prefill layout: one wave per (head slot, 4 consecutive token rows) ----
+// ---- prefill layout: one wave per (head slot, 4 NG consecutive token rows) ----
 //
-// Lane (g, j) = (lane / 16, lane % 16) handles token row r0 + g and the
-// channels c_i = 4j + i and c_{i+4} = 64 + 4j + i (i < 4), so RoPE partners
-// (c, c + 64) share a lane and every reduction over a row's 128 channels is a
-// 16-lane DPP row reduction. Compared with the one-wave-per-(row, head)
-// layout above, the per-row scalar chains (scale fits, divisors) run for four
-// rows at once and each head's scale vectors are loaded once per four rows.
+// Lane (g, j) = (lane / 16, lane % 16) handles token rows r0 + g NG + i, one
+// per pass i < NG, and the channels c_k = 4j + k and c_{k+4} = 64 + 4j + k (k
+// < 4), so RoPE partners (c, c + 64) share a lane and every reduction over a
+// row's 128 channels is a 16-lane DPP row reduction. Compared with the
+// one-wave-per-(row, head) layout above, the per-row scalar chains run for
+// four rows at once.
+//
+// What bounds it is the vector unit and, per row, the loads of the head's
+// scale vectors (int64, 3 x 8 per lane: six times the bytes of the row's own
+// product). NG rows per lane share them: they are loaded, checked and turned
+// into doubles once, the K divisors likewise, the next row's product and RoPE
+// entries load while the current row computes, the Q rows' DI-Exp constants
+// (one lane's serial chain) come from NG lanes side by side at the end, and a
+// lane's NG consecutive slots of V go out as one word instead of NG bytes.
+// Measured at 2048 rows of 32 heads (32 MB of product): 35.5 -> 26.0 us, vector
+// instructions 14.3 M -> 11.0 M (70 % of the issue slots), 4096 rows 64.2 ->
+// 44.7 us. The kinds are separate code (qkv_rows_kind), and rows outside the
+// fp64 forms' bounds are redone after the passes: either one inside the
+// passes costs enough registers to halve the waves in flight.
 // Same arithmetic and the same integers as qkv_head.
+typedef short v4s_u __attribute__((ext_vector_type(4), aligned(2)));  // any int16 alignment
+
+// The rows of the passes named in `bad` again, one at a time over the whole
+// wave (qkv_head: any operands), over what the fast passes stored. After the
+// passes, so that their registers are free.
+template <int NG>
+__device__ __forceinline__ void qkv_rows_redo(const QKVArgs& a, int R, int r0, int slotw,
+                                              uint32_t bad) {
+  __threadfence_block();  // the passes' stores are ahead of these
+  const int h = slotw < a.n_q ? slotw : 0;
+#pragma unroll 1
+  for (int q = 0; q < 4 * NG; ++q) {
+    const int r = r0 + q;
+    if (!((bad >> (q % NG)) & 1u) || r >= R) continue;
+    const int b = r / a.T, t = r - b * a.T;
+    const i64 qrow = ((i64)b * a.n_q + h) * a.T + t;
+    qkv_head(a, r, slotw, a.q8 + qrow * 128, a.tpos + qrow);
+  }
+}
 
 // The whole wave must be active. Rows r >= R compute on row R - 1 and store
-// nothing.
-__device__ __forceinline__ void qkv_rows4(const QKVArgs& a, int R, int r0, int slotw) {
+// nothing. KIND: the head slot's kind (0 query, 1 key, 2 value), so that each
+// kind holds its own operands only. Returns the passes (bit i) in which some
+// row left the fp64 forms' bounds: what they stored is redone (qkv_rows_redo).
+template <int NG, int KIND>
+__device__ __forceinline__ uint32_t qkv_rows_kind(const QKVArgs& a, int R, int r0, int slotw) {
+  static_assert(NG == 1 || NG == 4, "rows per lane");
   const int lane = threadIdx.x & 63, g = lane >> 4, j = lane & 15;
   const int n_heads = a.n_q + 2 * a.n_kv;
-  const bool rok = r0 + g < R;
-  const int r = rok ? r0 + g : R - 1;
-  const int b = r / a.T, t = r - b * a.T;
-  const i64 off = (i64)r * (n_heads * 128) + (i64)slotw * 128;
   const int group = a.n_q / a.n_kv;
-  const bool is_q = slotw < a.n_q, is_v = slotw >= a.n_q + a.n_kv;
+  constexpr bool is_q = KIND == 0, is_v = KIND == 2;
   const int h = is_q ? slotw : (is_v ? slotw - a.n_q - a.n_kv : slotw - a.n_q);
   const int kvh = is_q ? h / group : h;
+  const int rl = r0 + g * NG;  // this lane's first row
   int c[8];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     c[i] = 4 * j + i;
     c[i + 4] = 64 + 4 * j + i;
   }
-
-  // ---- loads
-  const i64 pos_raw = a.positions[r];
-  const i64 xk = a.xk[r], xm = a.xm[r];
-  const i64 base = slot_base_of(a);
-  // (candidates through opaque_ptr, as in qkv_head_load)
-  const int64_t* wmp =
-      (is_q ? opaque_ptr(a.q_m) : (is_v ? opaque_ptr(a.v_m) : opaque_ptr(a.k_m))) + (i64)h * 128;
-  // the head's column mantissas and product sums (loaded again by the
-  // integer routines, so the fp64 path does not keep them live)
-  auto load_wp = [&](i64 (&wm)[8], i64 (&p)[8]) {
-#pragma unroll
-    for (int i = 0; i < 8; ++i) wm[i] = ld_global(wmp + c[i]);
+  auto row = [&](int i) { return rl + i < R ? rl + i : R - 1; };
+  // a row's product sums (int32)
+  auto load_p = [&](int r, int32_t (&p)[8]) {
+    const i64 off = (i64)r * (n_heads * 128) + (i64)slotw * 128;
     uint32_t s[8] = {0, 0, 0, 0, 0, 0, 0, 0};
     for (int k = 0; k < a.nsplit; ++k) {
       const int32_t* pk = a.P + (i64)k * a.split_stride + off;
@@ -636,74 +678,117 @@ __device__ __forceinline__ void qkv_rows4(const QKVArgs& a, int R, int r0, int s
 #pragma unroll
     for (int i = 0; i < 8; ++i) p[i] = (int32_t)s[i];
   };
-  i64 wm[8], p[8];
-  load_wp(wm, p);
-  const i64 slot = base + t;
-  const int pg = rok ? a.kv.page(b, slot) : -1;
-  const bool sok = pg >= 0;
+  // the head's column mantissas
+  const int64_t* wmp = (is_q ? a.q_m : (is_v ? a.v_m : a.k_m)) + (i64)h * 128;
+  const int64_t* gam = is_q ? a.q_norm_m : a.k_norm_m;
+  const int64_t* qsp = a.qs_m + (i64)kvh * 128;
+  // (channels 4j + i of 16 lanes: contiguous 128-byte lines)
+  auto load8 = [&](const int64_t* v, i64 (&x)[8]) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) x[i] = ld_global(v + c[i]);
+  };
+  int32_t p[8];
+  load_p(row(0), p);
+  const i64 base = slot_base_of(a);
+  uint32_t bad = 0;  // bit i: pass i left the fp64 forms' bounds in some row (wave-uniform)
+  float wm[8];
+  bool hok = true;  // the head's mantissas are inside qk_head_f64's bounds
+  {
+    i64 w[8];
+    load8(wmp, w);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      hok = hok & in_range(w[i], QKV_WM_LIM);
+      wm[i] = (float)(int32_t)w[i];
+    }
+  }
+  // page of a row's slot (-1: not stored), its slot
+  auto place = [&](int i, i64* slot) {
+    const int r = row(i), b = r / a.T, t = r - b * a.T;
+    *slot = base + t;
+    return rl + i < R ? a.kv.page(b, *slot) : -1;
+  };
 
-  if (is_v) {
+  if constexpr (is_v) {
     // V head: requant_i8_static(Pv, xm, xk, v_m, v_k, vq_m[h], vq_k[h])
     const i64 vqm = a.vq_m[kvh], vqk = a.vq_k[kvh];
-    const i64 shift = wsub(wadd(xk, a.v_k), vqk);
-    const i64 up = imax(wneg(shift), 0), down = imax(shift, 0);
-    i64 den = shl(vqm, down);
-    if (den == 0) den = 1;  // the reference's division raises there
-    // n = P w_m x_m << up as an exact double: P w_m is one (|w_m| < 2^21) and
-    // the estimate's bound |n| < 2^49 leaves no room for a rounded product
-    // (one at or above 2^53 fails it); a lane outside runs the int64 form
-    constexpr i64 WM_LIM = (i64)1 << 21;
-    bool fast = den > 0 && den < ((i64)1 << 49);
-    const double xs = (double)xm * ldexp(1.0, (int)imin(up, 64));
-    double nd[8];
+    uint32_t word[8];  // byte i: pass i's value of channel c[k]
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      nd[i] = (double)(int32_t)p[i] * (double)(int32_t)wm[i] * xs;
-      fast = fast & in_range(wm[i], WM_LIM) & (fabs(nd[i]) < 0x1p49);
-    }
-    int8_t o[8];
-    if (DI_LIKELY(fast)) {
-      const DivEst D = make_divest(den, 1.0);
+    for (int k = 0; k < 8; ++k) word[k] = 0;
+#pragma unroll 1
+    for (int i = 0; i < NG; ++i) {
+      const int r = row(i);
+      const i64 xk = a.xk[r], xm = a.xm[r];
+      int32_t pn[8];
+      load_p(row(i + 1 < NG ? i + 1 : i), pn);
+      const i64 shift = wsub(wadd(xk, a.v_k), vqk);
+      const i64 up = imax(wneg(shift), 0), down = imax(shift, 0);
+      i64 den = shl(vqm, down);
+      if (den == 0) den = 1;  // the reference's division raises there
+      // n = P w_m x_m << up as int64 where its fp64 value (P w_m exact, |w_m| <
+      // 2^21, then one rounding) shows that no step wraps, its quotient from
+      // the corrected estimate (|n| passes the plain one's 2^49 in earnest: 24
+      // bits of P, 16 of each mantissa)
+      bool fast = hok & (den > 0) & (den < ((i64)1 << 52)) & (up < 62) & in_range(xm, (i64)1 << 40);
+      const int ups = up < 62 ? (int)up : 0;
+      const double xs = (double)xm * ldexp(1.0, ups);
+      const DivEst D = make_divest(fast ? den : 1, 1.0);
+      int o[8];
 #pragma unroll
-      for (int i = 0; i < 8; ++i) o[i] = (int8_t)rhad_est_i8_f64(nd[i], D);
-    } else {
-      i64 n[8];
+      for (int k = 0; k < 8; ++k) {
+        const double pw = (double)p[k] * mant_f64(wm[k]);
+        fast = fast & (fabs(pw * xs) < 0x1p61);
+        o[k] = rhad_est_i8_corr((i64)((u64)wmul((i64)pw, xm) << ups), den, D);
+      }
+      if (__ballot(!fast)) bad |= 1u << i;
 #pragma unroll
-      for (int i = 0; i < 8; ++i) n[i] = shl(wmul(wmul(p[i], wm[i]), xm), up);
-      if (den > 0) {
-        const Recip Rr = make_recip(den);
-#pragma unroll
-        for (int i = 0; i < 8; ++i) o[i] = (int8_t)clamp_i8(rhad_r(n[i], Rr));
-      } else {  // a wrapped, negative divisor: torch's floor division
-#pragma unroll
-        for (int i = 0; i < 8; ++i) o[i] = (int8_t)clamp_i8(rhad(n[i], den));
+      for (int k = 0; k < 8; ++k) {
+        word[k] |= (uint32_t)(uint8_t)(int8_t)o[k] << (8 * i);
+        p[k] = pn[k];
       }
     }
-    if (sok) {
+    // the lane's NG slots: one word when they are NG consecutive slots of one
+    // row that start at a multiple of NG (then they share a page too), else
+    // a byte each
+    const int b0 = row(0) / a.T;
+    i64 slot;
+    const int pg = place(0, &slot);
+    if (NG == 4 && rl + NG <= R && (rl + NG - 1) / a.T == b0 && (slot & (NG - 1)) == 0) {
+      if (pg >= 0) {
 #pragma unroll
-      for (int i = 0; i < 8; ++i) a.kv.vchan(pg, kvh, c[i])[slot & (DI_PAGE - 1)] = o[i];
+        for (int k = 0; k < 8; ++k)
+          *(uint32_t*)(a.kv.vchan(pg, kvh, c[k]) + (slot & (DI_PAGE - 1))) = word[k];
+      }
+    } else {
+#pragma unroll 1
+      for (int i = 0; i < NG; ++i) {
+        i64 sl;
+        const int pgi = place(i, &sl);
+        if (pgi >= 0) {
+#pragma unroll
+          for (int k = 0; k < 8; ++k)
+            a.kv.vchan(pgi, kvh, c[k])[sl & (DI_PAGE - 1)] = (int8_t)(word[k] >> (8 * i));
+        }
+      }
     }
-    return;
+    return bad;
   }
-  const int64_t* gam = is_q ? opaque_ptr(a.q_norm_m) : opaque_ptr(a.k_norm_m);
-  const i64 pos = torch_index(pos_raw, a.max_pos, (j == 0 && rok) ? a.err : nullptr,
-                              DI_ERR_POSITION);
-  // the head's gamma, RoPE and smoothing entries (loaded again by the
-  // integer routines)
-  auto load_ch = [&](i64 (&gm)[8], int32_t (&cs)[8], int32_t (&sn)[8], i64 (&qs)[8]) {
+
+  // the head's gamma and, as its kind needs, the smoothing mantissas (Q) or
+  // the static divisors (K, scaled by the numerator's up-shift: |r 2^up| r
+  // below is fma(|r|, 2^up r, k), an exact scaling)
+  float gm[8], qs[8];
+  double qa[8], kb[8];
+  double klim = 0.0;  // |r| below which every channel's divisor estimate holds
+  {
+    i64 w[8];
+    load8(gam, w);
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-      gm[i] = ld_global(gam + c[i]);
-      cs[i] = a.cos_t[pos * 128 + c[i]];
-      sn[i] = a.sin_t[pos * 128 + c[i]];
-      qs[i] = a.qs_m[kvh * 128 + c[i]];  // (unconditional: K heads ignore it)
+      hok = hok & in_range(w[i], QKV_G_LIM);
+      gm[i] = (float)(int32_t)w[i];
     }
-  };
-  i64 gm[8], qs[8];
-  int32_t cs[8], sn[8], p32[8];
-  load_ch(gm, cs, sn, qs);
-#pragma unroll
-  for (int i = 0; i < 8; ++i) p32[i] = (int32_t)p[i];
+  }
   const i64 rowk = 20 + a.k_norm_k;
   auto kq = [&](int i) -> KqChan {
     KqChan q;
@@ -718,138 +803,114 @@ __device__ __forceinline__ void qkv_rows4(const QKVArgs& a, int R, int r0, int s
     }
     return q;
   };
-  int o[8];
-  i64 am = 1;
-  const bool done = qk_head_f64<8, false>(is_q, p32, wm, gm, cs, sn, qs, kq, o, &am);
-  if (DI_UNLIKELY(!done)) {
-    // the integer routines (same integers, any operands)
-    i64 wm[8], p[8], gm[8], qs[8];
-    int32_t cs[8], sn[8];
-    load_wp(wm, p);
-    load_ch(gm, cs, sn, qs);
-    // requant_i32_common(tb = 16) per (token, head)   (model.py:207-211)
-    i64 y[8];
-    uint32_t L = 0;
+  if (is_q) {
+    i64 w[8];
+    load8(qsp, w);
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-      y[i] = wmul(p[i], wm[i]);
-      L = ::max(L, bitlen_abs(y[i]));
+      hok = hok & in_range(w[i], QKV_QS_LIM);
+      qs[i] = (float)(int32_t)w[i];
     }
-    {
-      const i64 sh = imax(ilog2_from_bitlen(row16_max_u32(L)) - 15, 0);
-      L = 0;
+  } else {
+    klim = 0x1p49;
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        y[i] = to_i32(rshift_round(y[i], sh));
-        L = ::max(L, bitlen_abs(y[i]));
-      }
+    for (int i = 0; i < 8; ++i) {
+      const KqChan q = kq(i);
+      const bool ok = q.den > 0 && q.den < ((i64)1 << 49) && q.up < 64;
+      const int up = ok ? (int)q.up : 0;
+      klim = fmin(klim, ok ? ldexp(0x1p49, -up) : -1.0);
+      qa[i] = ldexp(q.D.r, up);
+      kb[i] = q.D.k;
     }
-    // di_rmsnorm over the 128 channels (model.py:212)
-    {
-      const i64 sh = 25 - ilog2_from_bitlen(row16_max_u32(L));
-      const i64 up = imax(sh, 0), down = imax(-sh, 0);
-      i64 ss = 0;
+  }
+  auto kquant = [&](const double (&r)[8], int (&o)[8]) {
+    double m = 0.0;
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        y[i] = shl(rshift_round(y[i], down), up);
-        ss = wadd(ss, wmul(y[i], y[i]));
-      }
-      const i64 rms = imax(isqrt_est(rhad_pow2(row16_sum64(ss), 7)), 1);
-      if (DI_LIKELY(rms > ((i64)1 << 16))) {  // |y| <= 2^26 after the shift: rhad_est
-        const DivEst D = make_divest(rms, 1048576.0);
+    for (int i = 0; i < 8; ++i) m = fmax(m, fabs(r[i]));
 #pragma unroll
-        for (int i = 0; i < 8; ++i) y[i] = rhad_est_signed(y[i], D);
-      } else {
-        const Recip Rr = make_recip(rms);
-#pragma unroll
-        for (int i = 0; i < 8; ++i) y[i] = to_i32(rhad_r(shl(y[i], 20), Rr));
-      }
+    for (int i = 0; i < 8; ++i) o[i] = rhad_est_i8_f64(r[i], DivEst{qa[i], kb[i]});
+    return m < klim;
+  };
+  // RoPE entries of a row (4 at a time), reported once per row
+  auto load_rope = [&](int i, i64 pos_raw, v4s_u (&t)[4]) {
+    const i64 pos = torch_index(pos_raw, a.max_pos,
+                                (j == 0 && i < NG && rl + i < R) ? a.err : nullptr,
+                                DI_ERR_POSITION);
+    const int16_t* cp = a.cos_t + pos * 128 + 4 * j;
+    const int16_t* sp = a.sin_t + pos * 128 + 4 * j;
+    t[0] = *(const v4s_u*)cp;
+    t[1] = *(const v4s_u*)(cp + 64);
+    t[2] = *(const v4s_u*)sp;
+    t[3] = *(const v4s_u*)(sp + 64);
+  };
+  v4s_u rt[4];
+  load_rope(0, a.positions[row(0)], rt);
+  i64 am_keep = 1;
+#pragma unroll 1
+  for (int i = 0; i < NG; ++i) {
+    const int r = row(i);
+    // the next row's loads (the last pass loads its own row again)
+    int32_t pn[8];
+    v4s_u rn[4];
+    if (NG > 1) {
+      load_p(row(i + 1 < NG ? i + 1 : i), pn);
+      load_rope(i + 1, a.positions[row(i + 1 < NG ? i + 1 : i)], rn);
     }
+    int32_t cs[8], sn[8];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) y[i] = wmul(y[i], gm[i]);
-    // apply_int_rope at this token's position   (model.py:213-215; rope.py:38-55)
-    i64 rv[8];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      rv[i] = rshift_round(wadd(wmul(y[i], (i64)cs[i]), wmul(wneg(y[i + 4]), (i64)sn[i])), 14);
-      rv[i + 4] = rshift_round(wadd(wmul(y[i + 4], (i64)cs[i + 4]), wmul(y[i], (i64)sn[i + 4])), 14);
+    for (int k = 0; k < 4; ++k) {
+      cs[k] = rt[0][k];
+      cs[k + 4] = rt[1][k];
+      sn[k] = rt[2][k];
+      sn[k + 4] = rt[3][k];
     }
+    int o[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+    i64 am = 1;
+    const bool done = qk_head_f64<8, false>(is_q, p, wm, gm, cs, sn, qs, hok, kquant, o, &am);
+    if (__ballot(!done)) bad |= 1u << i;
+    uint32_t w[2] = {0, 0};
+#pragma unroll
+    for (int k = 0; k < 8; ++k) w[k >> 2] |= (uint32_t)(uint8_t)(int8_t)o[k] << (8 * (k & 3));
     if (!is_q) {
-      // K: requant_i8_static(kk, 1, k_rowk, 1, 0, kq_m, kq_k)   (model.py:326-329)
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const KqChan q = kq(i);
-        const i64 n = shl(rv[i], q.up);
-        const i64 lim = (i64)1 << 49;  // 2 |n| + den < 2^51 for rhad_est_i8
-        o[i] = (q.den > 0 && q.den < lim && n > -lim && n < lim) ? rhad_est_i8(n, q.D)
-                                                                 : (int)clamp_i8(rhad(n, q.den));
+      i64 slot;
+      const int pg = place(i, &slot);
+      if (pg >= 0) {
+        int8_t* krow = a.kv.krow(pg, h, (int)(slot & (DI_PAGE - 1)));
+        *(uint32_t*)(krow + 4 * j) = w[0];
+        *(uint32_t*)(krow + 64 + 4 * j) = w[1];
       }
     } else {
-      // Q: QK smoothing (model.py:317-320) then quant_i8_pertoken (model.py:322-323)
-      i64 q[8];
-      u64 amx = 0;  // unsigned: a q of INT64_MIN reads 2^63 (see the one-token form)
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        q[i] = wmul(rv[i], qs[i]);
-        amx = ::max(amx, (u64)wabs(q[i]));
+      const int b = r / a.T, t = r - b * a.T;
+      int8_t* qo = a.q8 + (((i64)b * a.n_q + h) * a.T + t) * 128;
+      if (rl + i < R) {
+        *(uint32_t*)(qo + 4 * j) = w[0];
+        *(uint32_t*)(qo + 64 + 4 * j) = w[1];
       }
-      constexpr u64 top = (u64)1 << 63;
-      const u64 amu = (u64)row16_max64((i64)(amx ^ top)) ^ top;
-      if (DI_LIKELY(amu < ((u64)1 << 43))) {  // as in quant_row: no 127 q wraps, 255 am < 2^51
-        am = imax((i64)amu, 1);
-        const DivEst D = make_divest(am, 127.0);
+      am_keep = j == i ? am : am_keep;
+    }
+    if (NG > 1) {
 #pragma unroll
-        for (int i = 0; i < 8; ++i) o[i] = rhad_est_signed(q[i], D);
-      } else {
-        if (DI_UNLIKELY(amu >> 63)) {  // uniform over the row's 16 lanes
-          i64 sx = 0;
+      for (int k = 0; k < 8; ++k) p[k] = pn[k];
 #pragma unroll
-          for (int i = 0; i < 8; ++i) sx = imax(sx, wabs(q[i]));
-          am = imax(row16_max64(sx), 1);
-        } else {
-          am = (i64)amu;
-        }
-        const Recip Rr = make_recip(am);
-#pragma unroll
-        for (int i = 0; i < 8; ++i) o[i] = (int)clamp_i8(rhad_r(wmul(q[i], 127), Rr));
-      }
+      for (int k = 0; k < 4; ++k) rt[k] = rn[k];
     }
   }
-  uint32_t w[2] = {0, 0};
-#pragma unroll
-  for (int i = 0; i < 8; ++i) w[i >> 2] |= (uint32_t)(uint8_t)(int8_t)o[i] << (8 * (i & 3));
-  if (!is_q) {
-    if (sok) {
-      int8_t* krow = a.kv.krow(pg, h, (int)(slot & (DI_PAGE - 1)));
-      *(uint32_t*)(krow + 4 * j) = w[0];
-      *(uint32_t*)(krow + 64 + 4 * j) = w[1];
-    }
-    return;
+  if (is_q && j < NG && rl + j < R) {
+    const int r = rl + j, b = r / a.T, t = r - b * a.T;
+    const i64 qrow = ((i64)b * a.n_q + h) * a.T + t;
+    a.tpos[qrow] = q_head_tpos(a, am_keep, a.ks_m[kvh], a.ks_k[kvh],
+                               a.dbg ? a.dbg + qrow * 4 : nullptr);
   }
-  const i64 qkk = 20 + a.q_norm_k + a.qs_k;
-  i64 m, k;
-  norm_scale(1, qkk, &m, &k);
-  const i64 qrow = ((i64)b * a.n_q + h) * a.T + t;
-  if (rok) {
-    *(uint32_t*)(a.q8 + qrow * 128 + 4 * j) = w[0];
-    *(uint32_t*)(a.q8 + qrow * 128 + 64 + 4 * j) = w[1];
-  }
-  if (j == 0 && rok) {
-    const i64 ksm = a.ks_m[kvh], ksk = a.ks_k[kvh];
-    i64 qm, e;
-    fit_dyadic_ratio_127(wmul(am, m), &qm, &e);
-    const i64 qk = wadd(k, e);
-    // score scale: norm_scale(qm * ks_m[h//g], qk + ks_k[h//g])   (model.py:351-353)
-    i64 sm, sk;
-    norm_scale(wmul(qm, ksm), wadd(qk, ksk), &sm, &sk);
-    a.tpos[qrow] = di_exp_tpos_fast(sm, sk);
-    if (a.dbg) {
-      a.dbg[qrow * 4 + 0] = qm;
-      a.dbg[qrow * 4 + 1] = qk;
-      a.dbg[qrow * 4 + 2] = sm;
-      a.dbg[qrow * 4 + 3] = sk;
-    }
-  }
+  return bad;
+}
+
+template <int NG>
+__device__ __forceinline__ void qkv_rows(const QKVArgs& a, int R, int r0, int slotw) {
+  uint32_t bad;
+  if (slotw < a.n_q) bad = qkv_rows_kind<NG, 0>(a, R, r0, slotw);
+  else if (slotw < a.n_q + a.n_kv) bad = qkv_rows_kind<NG, 1>(a, R, r0, slotw);
+  else bad = qkv_rows_kind<NG, 2>(a, R, r0, slotw);
+  if (DI_UNLIKELY(bad != 0)) qkv_rows_redo<NG>(a, R, r0, slotw, bad);
 }
 
 }  // namespace di

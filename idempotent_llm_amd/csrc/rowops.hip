@@ -1116,19 +1116,20 @@ __global__ __launch_bounds__(RT) void k_qkv_epilogue(QKVArgs a) {
   qkv_head(a, r, slotw, a.q8 + qrow * 128, a.tpos + qrow);
 }
 
-// Many token rows (prefill): one wave per (head slot, 4 rows), head-major so
-// a block's waves share a head's scale vectors.
-#ifndef QKV_ROWS_MINW
-#define QKV_ROWS_MINW 1
-#endif
-__global__ __launch_bounds__(RT, QKV_ROWS_MINW) void k_qkv_epilogue_rows(QKVArgs a, int R, int ngroups) {
+// Many token rows (prefill): one wave per (head slot, 4 NG rows), head-major
+// so a block's waves share a head's scale vectors. Registers: at NG = 4 a
+// wave lives for four passes, and four waves per SIMD (128 VGPRs) keep the
+// vector unit busy; at NG = 1 three waves without spills beat four with them.
+template <int NG>
+__global__ __launch_bounds__(RT, NG == 4 ? 4 : 3) void k_qkv_epilogue_rows(QKVArgs a, int R,
+                                                                           int ngroups) {
   keep_hidden_args();
   const int heads = a.n_q + 2 * a.n_kv;
   // (wave-uniform, so the head slot's pointer and scale selects stay scalar)
   const int wg = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * 4 + (threadIdx.x >> 6)));
   if (wg >= heads * ngroups) return;  // whole waves only
   const int slotw = wg / ngroups, grp = wg - slotw * ngroups;
-  qkv_rows4(a, R, grp * 4, slotw);
+  qkv_rows<NG>(a, R, grp * 4 * NG, slotw);
 }
 
 // Bookkeeping of one graphed decode step before its replay (graphed.py:112-131
@@ -2214,11 +2215,20 @@ int detllm_qkv_epilogue(const int32_t* P, int nsplit, int64_t split_stride, int 
   const int R = B * T;
   // the rows layout reads P 16 bytes at a time
   if (R > 64 && (nsplit == 1 || split_stride % 4 == 0) && ((uintptr_t)P & 15) == 0) {
-    const int ngroups = (R + 3) / 4;
+    // Rows per lane: four once the launch has about a round of waves left at
+    // four rows per lane (36864 (row, head) pairs, 1152 rows of 32 heads: two
+    // waves per SIMD), where sharing the scale vectors pays; below, one row
+    // per lane and four times the waves. Measured at 32 heads, four against
+    // one: 200 rows 14.9 / 7.7 us, 1024 rows 18.9 / 18.3, 1200 rows 20.9 /
+    // 22.7, 2048 rows 26.0 / 35.4.
+    const bool many = (i64)R * heads >= 36864;
+    const int rows = many ? 16 : 4;
+    const int ngroups = (R + rows - 1) / rows;
     const i64 waves = (i64)ngroups * heads;
-    if ((waves + 3) / 4 > 0x7fffffff) return DI_ERANGE;
-    hipLaunchKernelGGL(k_qkv_epilogue_rows, dim3((unsigned)((waves + 3) / 4)), dim3(RT), 0, s, a,
-                       R, ngroups);
+    if (waves > 0x7fffffff) return DI_ERANGE;
+    const dim3 grid((unsigned)((waves + 3) / 4));
+    if (many) hipLaunchKernelGGL(k_qkv_epilogue_rows<4>, grid, dim3(RT), 0, s, a, R, ngroups);
+    else hipLaunchKernelGGL(k_qkv_epilogue_rows<1>, grid, dim3(RT), 0, s, a, R, ngroups);
   } else {
     hipLaunchKernelGGL(k_qkv_epilogue, dim3(R, (heads + 3) / 4), dim3(RT), 0, s, a);
   }

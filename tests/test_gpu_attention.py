@@ -606,3 +606,53 @@ def test_qkv_epilogue_every_path(variant, B, T):
         k, v = unpaged(ka, va, table, S)
         np.testing.assert_array_equal(k[:, :, slot].cpu().numpy(), want_k[:, :, 0])
         np.testing.assert_array_equal(v[:, :, slot].cpu().numpy(), want_v[:, :, 0])
+
+
+@pytest.mark.parametrize("variant", ["none", "ranges", "gamma"])
+@pytest.mark.parametrize("B,T,slot", [(3, 401, 0), (2, 640, 128), (5, 256, 3), (1, 1153, 126)])
+def test_qkv_epilogue_rows_per_lane(variant, B, T, slot):
+    """The epilogue of many rows (four rows per lane) against the oracle: a
+    last group of fewer rows, groups that cross a batch row or a page, V slots
+    that start inside a word, and heads and rows that leave the fp64 forms
+    (_plant's channels, a zero head, a row whose V numerators wrap)."""
+    from idempotent_llm_amd._lib import call
+    print(f"[qkv epilogue rows per lane {variant} B={B} T={T} slot={slot}]", flush=True)
+    dims = art.MID
+    nq, nkv, hd = dims["n_q_heads"], dims["n_kv_heads"], 128
+    prm = _plant(_layer_params(dims, 6), variant, nq, nkv)
+    R = B * T
+    assert R * (nq + 2 * nkv) >= 36864
+    rnd = torch.Generator().manual_seed(B * 1000 + T)
+    P = torch.randint(-(1 << 19), 1 << 19, (1, R, (nq + 2 * nkv) * hd), generator=rnd,
+                      dtype=torch.int32)
+    P[0, 5, 9 * hd:10 * hd] = 0
+    P[0, R - 1, (nq + 6) * hd:(nq + 7) * hd] = 0
+    P = P.cuda()
+    xm = torch.randint(1 << 15, 1 << 16, (R,), generator=rnd, dtype=I64)
+    xm[R // 2] = (1 << 40) + 7
+    xm = xm.cuda()
+    xk = torch.randint(22, 30, (R,), generator=rnd, dtype=I64).cuda()
+    pos = torch.randint(0, dims["max_pos"], (R,), generator=rnd, dtype=I64).cuda()
+    want_q8, want_tpos, want_k, want_v, _ = _qkv_oracle(P, xm, xk, pos, prm, B, T, nq, nkv)
+    cap = slot + T
+    for nsplit in (1, 2):     # and the product as two partials
+        Ps = P if nsplit == 1 else torch.cat([P - 12345, torch.full_like(P, 12345)])
+        q8 = torch.full((B, nq, T, hd), 99, dtype=torch.int8, device="cuda")
+        tpos = torch.full((B, nq, T), -1, dtype=I64, device="cuda")
+        k0 = torch.randint(-128, 128, (B, nkv, cap, hd), generator=rnd, dtype=torch.int8)
+        v0 = torch.randint(-128, 128, (B, nkv, hd, cap), generator=rnd, dtype=torch.int8)
+        kc, vc, table, width = paged(k0, v0, seed=T)
+        call("detllm_qkv_epilogue", Ps, nsplit, R * P.shape[2], B, T, nq, nkv, xm, xk, pos,
+             prm["q_m"], prm["q_k"], prm["k_m"], prm["k_k"], prm["v_m"], prm["v_k"],
+             prm["q_norm_m"], prm["q_norm_k"], prm["k_norm_m"], prm["k_norm_k"], prm["qs_m"],
+             prm["qs_k"], prm["kq_m"], prm["kq_k"], prm["ks_m"], prm["ks_k"], prm["vq_m"],
+             prm["vq_k"], prm["cos"], prm["sin"], prm["cos"].shape[0], q8, tpos, None, kc, vc,
+             table, width, None, slot, None, None)
+        torch.cuda.synchronize()
+        k, v = unpaged(kc, vc, table, cap)
+        np.testing.assert_array_equal(q8.cpu().numpy(), want_q8)
+        np.testing.assert_array_equal(tpos.cpu().numpy(), want_tpos)
+        np.testing.assert_array_equal(k[:, :, slot:].cpu().numpy(), want_k)
+        np.testing.assert_array_equal(v[:, :, slot:].cpu().numpy(), want_v)
+        assert torch.equal(k[:, :, :slot].cpu(), k0[:, :, :slot])   # earlier slots untouched
+        assert torch.equal(v[:, :, :slot].cpu(), v0.transpose(2, 3)[:, :, :slot])

@@ -511,6 +511,34 @@ def test_rhad_est_signed_i8_and_corrected(lib):
     assert got.tolist() == [rh(127 * a, d) for a, d in zip(A, D)]
 
 
+def test_rhad_est_i8_corrected(lib):
+    """The int8-clamped division with the remainder step (the V heads' static
+    requantisation) against exact rhad in Python integers: |n| < 2^62, d <
+    2^52, ties and their neighbours at every quotient around and past the
+    clamp, and numerators of every size."""
+    rnd = random.Random(31)
+
+    def rh(a, d):
+        q = (abs(a) + d // 2) // d
+        return max(-128, min(127, -q if a < 0 else q))
+
+    lim = (1 << 62) - 1
+    A, D = [], []
+    for _ in range(8000):
+        d = rnd.randrange(1, 1 << rnd.randrange(1, 53))
+        q = rnd.choice([0, 1, 126, 127, 128, 129, 253, 254, 255, 256, rnd.randrange(0, 300)])
+        t = q * d - d // 2
+        for a in (t - 1, t, t + 1, q * d, rnd.randrange(0, 1 << rnd.randrange(1, 63)), lim):
+            A.append(min(max(a, 0), lim) * rnd.choice([1, -1]))
+            D.append(d)
+    for d in (1, 2, 3, (1 << 52) - 1, 1 << 51):
+        for a in (0, 1, -1, d // 2, (d + 1) // 2, 127 * d + d // 2, 128 * d, 255 * d - 1, -lim):
+            A.append(max(min(a, lim), -lim))
+            D.append(d)
+    got = _est_op(lib, 3, A, D, [1] * len(A))
+    assert got.tolist() == [rh(a, d) for a, d in zip(A, D)]
+
+
 def test_isqrt_est_matches_oracle(lib):
     """isqrt_est (fp64 square root + one integer step each way) equals the
     oracle's isqrt (int_prims.py bitwise method) below 2^62: random values at
