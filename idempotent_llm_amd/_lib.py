@@ -1,4 +1,6 @@
-"""ctypes binding of libdetllm_hip.so (the extern "C" boundary).
+"""Binding of libdetllm_hip.so (the extern "C" boundary): ``call`` goes
+through the native thunks of ``_native.so`` (csrc/torch_binding.cpp), the
+host-only planners through ctypes.
 
 Every entry point takes device pointers, sizes and a hipStream_t and returns
 0 on success, a positive hipError_t for a failed launch or a negative errno
@@ -10,12 +12,14 @@ loudly.
 from __future__ import annotations
 
 import ctypes
+import importlib
 import os
 
 import torch
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libdetllm_hip.so")
+NATIVE_PATH = os.path.join(_HERE, "_native.so")
 
 P, I, L, S = "p", "i", "l", "s"
 
@@ -75,10 +79,24 @@ HOST_ONLY = frozenset({"detllm_igemv_plan", "detllm_attn_split_plan"})
 _CT = {P: ctypes.c_void_p, I: ctypes.c_int, L: ctypes.c_int64, S: ctypes.c_void_p}
 
 _lib = None
+_entries: dict = {}   # name -> native callable entry(stream, *args)
 
 
 class LibraryMissing(RuntimeError):
     pass
+
+
+def _missing(path):
+    return LibraryMissing(
+        f"{path} is not built; run `python -c 'import __graft_entry__ as g; g.build()'` "
+        "(the rocm backend has no CPU fallback)")
+
+
+def native():
+    """The native binding module (raises LibraryMissing when it is not built)."""
+    if not os.path.exists(NATIVE_PATH):
+        raise _missing(NATIVE_PATH)
+    return importlib.import_module(__package__ + "._native")
 
 
 def load():
@@ -87,28 +105,15 @@ def load():
     if _lib is not None:
         return _lib
     if not os.path.exists(LIB_PATH):
-        raise LibraryMissing(
-            f"{LIB_PATH} is not built; run `python -c 'import __graft_entry__ as g; g.build()'` "
-            "(the rocm backend has no CPU fallback)")
+        raise _missing(LIB_PATH)
     lib = ctypes.CDLL(LIB_PATH)
     for name, kinds in SIGNATURES.items():
         fn = getattr(lib, name)
         fn.argtypes = [_CT[k] for k in kinds]
         fn.restype = ctypes.c_int
+    _entries.update(native().entries())
     _lib = lib
     return lib
-
-
-def _arg(kind, v):
-    if kind == P:
-        if v is None:
-            return None
-        if isinstance(v, torch.Tensor):
-            return v.data_ptr()
-        return int(v)
-    if kind == S:
-        return v
-    return int(v)
 
 
 def stream_handle(stream=None) -> int:
@@ -173,14 +178,8 @@ def raise_for_error_word(word: int, vocab=None, max_pos=None) -> None:
 
 
 def call(name: str, *args, stream=None) -> None:
-    """Invoke an entry point; tensors are passed by device pointer and the
-    current torch stream is appended as the hipStream_t argument."""
-    lib = load()
-    kinds = SIGNATURES[name]
-    if len(args) != len(kinds) - 1:
-        raise TypeError(f"{name}: expected {len(kinds) - 1} arguments, got {len(args)}")
-    cargs = [_arg(k, v) for k, v in zip(kinds[:-1], args)]
-    cargs.append(stream_handle(stream))
-    rc = getattr(lib, name)(*cargs)
-    if rc != 0:
-        raise RuntimeError(f"{name} failed (code {rc})")
+    """Invoke an entry point; tensors are passed by device pointer and torch's
+    current stream (or the given torch stream) as the hipStream_t argument."""
+    if _lib is None:
+        load()
+    _entries[name](None if stream is None else stream.cuda_stream, *args)

@@ -42,15 +42,6 @@ def _require_rocm(backend: str):
         raise ValueError(f"unknown backend {backend!r}")
 
 
-def _pad_k(x: torch.Tensor, Kp: int) -> torch.Tensor:
-    K = x.shape[-1]
-    if K == Kp:
-        return x.contiguous()
-    out = torch.zeros(*x.shape[:-1], Kp, dtype=x.dtype, device=x.device)
-    out[..., :K] = x
-    return out
-
-
 def transpose_i8(b: torch.Tensor) -> torch.Tensor:
     """[*, R, C] int8 -> [*, C, R] on the device (HIP transpose kernel)."""
     R, C = b.shape[-2], b.shape[-1]
@@ -92,28 +83,6 @@ def int_gemm(a: torch.Tensor, b: torch.Tensor, backend: str = "rocm") -> torch.T
     if b.dim() != 2 or a.dim() == 2:
         assert a.shape[:-2] == b.shape[:-2], (a.shape, b.shape)
     return torch.ops.detllm_rocm.int_gemm(a, b)
-
-
-def _int_gemm_impl(a: torch.Tensor, b: torch.Tensor) -> torch.Tensor:
-    """The kernel behind detllm_rocm::int_gemm (operands checked by int_gemm)."""
-    if b.dim() == 2 and a.dim() > 2:
-        lead = a.shape[:-1]
-        out = _int_gemm_impl(a.reshape(-1, a.shape[-1]), b)
-        return out.reshape(*lead, b.shape[-1])
-    M, K, N = a.shape[-2], a.shape[-1], b.shape[-1]
-    if M == 0 or N == 0:
-        return torch.zeros(*a.shape[:-1], N, dtype=torch.int32, device=a.device)
-    Kp = max(16, (K + 15) // 16 * 16)
-    bt = _pad_k(transpose_i8(b), Kp)
-    ap = _pad_k(a, Kp)
-    if a.dim() == 2:
-        return gemm_nt(ap, bt)[0]
-    A = ap.reshape(-1, M, Kp)
-    Bt = bt.reshape(-1, N, Kp)
-    batch = A.shape[0]
-    out = torch.empty(batch, M, N, dtype=torch.int32, device=a.device)
-    call("detllm_igemm_nt", A, Bt, out, M, N, Kp, batch, M * Kp, N * Kp, M * N)
-    return out.reshape(*a.shape[:-2], M, N)
 
 
 def int_gemm_u8i8(p_u8: torch.Tensor, b: torch.Tensor, backend: str = "rocm") -> torch.Tensor:

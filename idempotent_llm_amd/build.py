@@ -2,6 +2,8 @@
 
 ``libdetllm_hip.so``      — every kernel + the extern "C" boundary
                             (declared in include/detllm_hip.h);
+``_native.so``            — the entry points as Python callables and torch
+                            operators (csrc/torch_binding.cpp);
 ``libdetllm_intops_host.so`` — intops.h compiled for the CPU, used by the
                             CPU test suite to check the integer routines the
                             kernels share.
@@ -23,6 +25,7 @@ PKG = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(PKG, "csrc")
 BUILD = os.path.join(os.path.dirname(PKG), "_build")
 LIB = os.path.join(PKG, "libdetllm_hip.so")
+NATIVE = os.path.join(PKG, "_native.so")
 HOST_LIB = os.path.join(PKG, "libdetllm_intops_host.so")
 HIP_SOURCES = ("gemm.hip", "rowops.hip", "attention.hip")
 ARCH = "gfx950"
@@ -61,8 +64,31 @@ def build(verbose: bool = False) -> str:
     tmp = LIB + ".tmp"
     _run([hipcc, "-shared", f"--offload-arch={ARCH}", "-fPIC", *objs, "-o", tmp])
     os.replace(tmp, LIB)
+    build_native()
     build_host_shim()
     return LIB
+
+
+def build_native() -> str:
+    """The Python / torch binding, linked against the library just built
+    (found next to it) and torch's own libraries (loaded by ``import torch``)."""
+    import sysconfig
+
+    import torch
+    gxx = shutil.which("g++") or "g++"
+    root = os.path.dirname(torch.__file__)
+    inc = [os.path.join(root, "include"),
+           os.path.join(root, "include", "torch", "csrc", "api", "include"),
+           sysconfig.get_paths()["include"],
+           os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "include")]
+    tmp = NATIVE + ".tmp"
+    _run([gxx, "-O2", "-std=c++17", "-shared", "-fPIC", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",
+          f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+          *(f"-I{d}" for d in inc), os.path.join(CSRC, "torch_binding.cpp"), "-o", tmp,
+          "-L" + os.path.join(root, "lib"), "-ltorch_python", "-ltorch_cpu", "-lc10", "-lc10_hip",
+          "-L" + PKG, "-l:libdetllm_hip.so", "-Wl,-rpath,$ORIGIN"])
+    os.replace(tmp, NATIVE)
+    return NATIVE
 
 
 def build_host_shim() -> str:

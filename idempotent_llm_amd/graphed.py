@@ -115,10 +115,10 @@ class GraphedDecode:
         return logits
 
     def _capture(self):
-        # warm-up: real executions of this same step (idempotent: they write
-        # the same K/V bytes to the same slot)
-        for _ in range(3):
-            self._run()
+        # warm-up: one real execution of this same step (idempotent: it writes
+        # the same K/V bytes to the same slot), so that every kernel of the
+        # step is loaded before the capture
+        self._run()
         torch.cuda.synchronize()
         g = torch.cuda.CUDAGraph()
         with torch.cuda.graph(g):
@@ -128,8 +128,7 @@ class GraphedDecode:
     def _capture_pick(self):
         # warm-up as in _capture (the forward only: the pick would overwrite
         # this step's input ids), then one graph of the forward and the pick
-        for _ in range(3):
-            self._run()
+        self._run()
         torch.cuda.synchronize()
         g = torch.cuda.CUDAGraph()
         with torch.cuda.graph(g):

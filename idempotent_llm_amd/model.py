@@ -95,6 +95,15 @@ class LayerWeights:
     # per-channel divisors of the static K requantisation, [n_kv * 128, 4]
     # int64 (detllm_kq_est): layer constants computed once at load
     kq_est: torch.Tensor | None = None
+    # the model's RoPE tables and their size (cos, sin, max_pos)
+    rope: tuple = ()
+
+    @property
+    def epi(self) -> tuple:
+        """The Q/K/V epilogue's layer constants in its argument order."""
+        return (self.q_m, self.q_k, self.k_m, self.k_k, self.v_m, self.v_k, self.q_norm_m,
+                self.q_norm_k, self.k_norm_m, self.k_norm_k, self.qs_m, self.qs_k, self.kq_m,
+                self.kq_k, self.ks_m, self.ks_k, self.vq_m, self.vq_k, *self.rope)
 
     # the reference's field names (model.py:41-64) as views of the kernel
     # layout, for code written against the reference class (seam overrides)
@@ -130,6 +139,24 @@ class LayerWeights:
     @property
     def k_rowk(self) -> int:
         return OUT_FRAC_BITS + self.k_norm_k
+
+
+class _Workspace(dict):
+    """The buffers of one forward pass by name: made at their first use and
+    used again by every later layer of the pass (launches of one pass run in
+    order on one stream, so a buffer's readers are ahead of its next writer).
+    A pass makes its own, so concurrent passes share nothing."""
+
+    def __init__(self, device):
+        super().__init__()
+        self.device = device
+        self.valid = None      # the cache's validity mask as bytes
+
+    def buf(self, name, shape, dtype):
+        t = self.get(name)
+        if t is None:
+            t = self[name] = torch.empty(shape, dtype=dtype, device=self.device)
+        return t
 
 
 def _pack(L: LayerWeights, names) -> torch.Tensor:
@@ -229,6 +256,7 @@ class IntQwen3:
             L.pf_mlp = _pack(L, ["gate_m", "up_m", "ds_m"])
             L.kq_est = torch.empty(L.kq_m.numel(), 4, dtype=I64, device=dev)
             call("detllm_kq_est", L.kq_m, L.kq_k, L.kq_m.numel(), 20 + L.k_norm_k, L.kq_est)
+            L.rope = (self.rope_cos, self.rope_sin, self.max_pos)
         self._greedy_scratch = {}
         self._plans: dict = {}
         self._split_plans: dict = {}
@@ -293,17 +321,20 @@ class IntQwen3:
         N, K = w.shape
         return (w, N, K, self._ksplit(N, K, R))
 
-    def _gemm(self, x: torch.Tensor, w: torch.Tensor, prefetch=(), split: bool = True):
+    def _gemm(self, x: torch.Tensor, w: torch.Tensor, prefetch=(), split: bool = True,
+              ws: _Workspace | None = None, name: str = ""):
         """x . w^T as int32 partials [ks, R, N] (ks = 1 unless split and the
         skinny GEMM's plan splits K). prefetch: up to four device tensors the
         next kernels read; the skinny GEMM pulls them into the memory-side
-        cache while it streams w (a hint, results unchanged)."""
+        cache while it streams w (a hint, results unchanged). With ws the
+        partials are its buffer `name`."""
         R, K = x.shape
         N = w.shape[0]
+        ks = self._ksplit(N, K, R) if split and R <= 64 else 1
+        P = (torch.empty(ks, R, N, dtype=torch.int32, device=self.device) if ws is None
+             else ws.buf(name, (ks, R, N), torch.int32))
         if R > 64:
-            return gemm_nt(x, w), 1, R * N
-        ks = self._ksplit(N, K, R) if split else 1
-        P = torch.empty(ks, R, N, dtype=torch.int32, device=self.device)
+            return gemm_nt(x, w, out=P), 1, R * N
         pf = []
         for t in prefetch[:4]:
             pf += [t, t.numel() * t.element_size()]
@@ -362,12 +393,14 @@ class IntQwen3:
         call("detllm_embed_normq", ids.contiguous().view(-1), R, H, self.vocab, self.embed_e8,
              self.embed_m, self.embed_k, h, k_res, L0.as_m, L0.as_k, x8, xm, xk, self._err)
         pos = positions.contiguous().view(-1)
+        ws = _Workspace(dev)
+        ws.valid = cache.valid_buf.view(torch.uint8)
         if fused:
-            self._layers_fused(B, hb, kb, x8, xm, xk, pos, cache, S_past, S, static)
+            self._layers_fused(ws, B, hb, kb, x8, xm, xk, pos, cache, S_past, S, static)
         else:
             for li, L in enumerate(self.layers):
                 nxt = self.layers[li + 1] if li + 1 < self.n_layers else None
-                self._layer(L, nxt, B, T, h, k_res, x8, xm, xk, pos, cache, S_past, S, static)
+                self._layer(ws, L, nxt, B, T, h, k_res, x8, xm, xk, pos, cache, S_past, S, static)
         if not static:
             cache.length = S
         if head_rows is not None:
@@ -445,11 +478,11 @@ class IntQwen3:
         pos = positions.view(B, 1, T).expand(B, n_heads, T)
         return ops.apply_int_rope(yn, self.rope_cos, self.rope_sin, pos), k_out
 
-    def _layer(self, L: LayerWeights, nxt, B, T, h, k_res, x8, xm, xk, pos, cache: KVCache,
-               S_past, S, static):
-        P, ns, st = self._gemm(x8, L.wqkv, (L.pf_attn,))
-        attn = self._attend(L, B, T, P, ns, st, xm, xk, pos, cache, S_past, S, static)
-        self._after_attention(L, nxt, B, T, attn, h, k_res, x8, xm, xk)
+    def _layer(self, ws: _Workspace, L: LayerWeights, nxt, B, T, h, k_res, x8, xm, xk, pos,
+               cache: KVCache, S_past, S, static):
+        P, ns, st = self._gemm(x8, L.wqkv, (L.pf_attn,), ws=ws, name="P_qkv")
+        attn = self._attend(ws, L, B, T, P, ns, st, xm, xk, pos, cache, S_past, S, static)
+        self._after_attention(ws, L, nxt, B, T, attn, h, k_res, x8, xm, xk)
 
     def _split_plan(self, B: int, S: int):
         """(chunk, nsplit) of the split-S decode attention, or None when the
@@ -464,65 +497,60 @@ class IntQwen3:
             self._split_plans[key] = plan
         return plan if plan[1] > 1 else None
 
-    def _attend(self, L: LayerWeights, B, T, P, ns, st, xm, xk, pos, cache: KVCache, S_past, S,
-                static):
+    def _attend(self, ws: _Workspace, L: LayerWeights, B, T, P, ns, st, xm, xk, pos,
+                cache: KVCache, S_past, S, static):
         """Q/K/V epilogue (cache write) and attention of one layer from the
         QKV partials P. Returns (attn, nsplit, split_stride, ext): int64
         context partials [nsplit][B * T][n_q * hd] whose sum is the context,
         and the merge statistics [B][n_kv][2] of a decode step's context
         (detllm_qkv_attn_decode_ext), else None."""
-        dev = self.device
         R, nq, nkv, hd = B * T, self.n_q, self.n_kv, self.hd
         li = L.idx
-        valid = cache.valid_buf.view(torch.uint8)
+        valid = ws.valid
         plan = self._split_plan(B, S) if T == 1 else None
         if plan is not None:
             # long rows: Q/K/V epilogue, then the split-S attention
             chunk, nsp = plan
-            q8 = torch.empty(B, nq, 1, hd, dtype=torch.int8, device=dev)
-            tpos = torch.empty(B, nq, 1, dtype=I64, device=dev)
+            q8 = ws.buf("q8", (B, nq, 1, hd), torch.int8)
+            tpos = ws.buf("tpos", (B, nq, 1), I64)
             call("detllm_qkv_epilogue", P, ns, st, B, 1, nq, nkv, xm, xk, pos,
-                 L.q_m, L.q_k, L.k_m, L.k_k, L.v_m, L.v_k, L.q_norm_m, L.q_norm_k,
-                 L.k_norm_m, L.k_norm_k, L.qs_m, L.qs_k, L.kq_m, L.kq_k, L.ks_m, L.ks_k,
-                 L.vq_m, L.vq_k, self.rope_cos, self.rope_sin, self.max_pos, q8, tpos, None,
+                 *L.epi, q8, tpos, None,
                  *cache.layer_args(li), cache.len_idx if static else None,
                  0 if static else S_past, L.kq_est, self._err)
-            scores = torch.empty(B, nq, nsp * chunk, dtype=torch.int32, device=dev)
-            cmax = torch.empty(B, nq, nsp, dtype=torch.int32, device=dev)
-            attn = torch.empty(nsp, R, nq * hd, dtype=I64, device=dev)
+            scores = ws.buf("scores", (B, nq, nsp * chunk), torch.int32)
+            cmax = ws.buf("cmax", (B, nq, nsp), torch.int32)
+            attn = ws.buf("attn", (nsp, R, nq * hd), I64)
             call("detllm_attn_decode_split", q8, tpos, *cache.layer_args(li), valid, cache.cap,
                  B, S, nq, nkv, cache.nslots if static else None, chunk, scores, cmax, attn,
                  self._err)
             return attn, nsp, R * nq * hd, None
-        attn = torch.empty(R, nq * hd, dtype=I64, device=dev)
+        attn = ws.buf("attn", (R, nq * hd), I64)
         if T == 1 and nq // nkv <= 2:
             # decode: Q/K/V epilogue and attention in one launch
-            scratch = self._decode_scratch(B, S)
+            scratch = self._decode_scratch(ws, B, S)
             args = (P, ns, st, B, nq, nkv, xm, xk, pos,
-                    L.q_m, L.q_k, L.k_m, L.k_k, L.v_m, L.v_k, L.q_norm_m, L.q_norm_k,
-                    L.k_norm_m, L.k_norm_k, L.qs_m, L.qs_k, L.kq_m, L.kq_k, L.ks_m, L.ks_k,
-                    L.vq_m, L.vq_k, self.rope_cos, self.rope_sin, self.max_pos,
+                    *L.epi,
                     *cache.layer_args(li), cache.len_idx if static else None,
                     0 if static else S_past, valid, cache.cap, S,
                     cache.nslots if static else None, scratch, attn, self._err)
             if B <= MERGE_EXT_ROWS and nq * hd <= 2048 and nkv <= 8:
                 # with the merge's row statistics, for the o-GEMV that
                 # quantises its own K range of the operand
-                ext = torch.empty(B, nkv, 2, dtype=I64, device=dev)
+                ext = ws.buf("ext", (B, nkv, 2), I64)
                 call("detllm_qkv_attn_decode_ext", *args, L.osc_m, ext)
                 return attn, 1, 0, ext
             call("detllm_qkv_attn_decode", *args)
         elif T > 1 and self._seams_overridden():
             self._attention_seams(L, B, T, P, ns, st, xm, xk, pos, cache, S_past, S, attn)
         else:
-            self._attention(L, B, T, P, ns, st, xm, xk, pos, cache, S_past, S, static, attn)
+            self._attention(ws, L, B, T, P, ns, st, xm, xk, pos, cache, S_past, S, static, attn)
         return attn, 1, 0, None
 
-    def _partials(self, R: int, N: int, K: int):
+    def _partials(self, ws: _Workspace, name: str, R: int, N: int, K: int):
         ks = self._ksplit(N, K, R)
-        return torch.empty(ks, R, N, dtype=torch.int32, device=self.device), ks, R * N
+        return ws.buf(name, (ks, R, N), torch.int32), ks, R * N
 
-    def _layers_fused(self, B, hb, kb, x8, xm, xk, pos, cache, S_past, S, static):
+    def _layers_fused(self, ws: _Workspace, B, hb, kb, x8, xm, xk, pos, cache, S_past, S, static):
         """The decoder stack for a decode row (T == 1, B == 1) with each
         skinny GEMM's operand row kernel fused into it (detllm_igemv_merge,
         detllm_igemv_resnormq, detllm_igemv_swiglu): per layer
@@ -533,20 +561,16 @@ class IntQwen3:
         between two buffers (a fused launch reads one while its lead block
         writes the other): hb [2, B, H], kb [2, B] with the embedding's
         residual in buffer 0."""
-        dev = self.device
         R, H, nq, hd, I_ = B, self.hidden, self.n_q, self.hd, self.inter
         cur = 0
-        am = torch.empty(R, dtype=I64, device=dev)
-        ak = torch.empty(R, dtype=I64, device=dev)
-        y8 = torch.empty(R, I_, dtype=torch.int8, device=dev)
-        ym = torch.empty(R, dtype=I64, device=dev)
-        yk = torch.empty(R, dtype=I64, device=dev)
+        am, ak, ym, yk = (ws.buf(n, (R,), I64) for n in ("am", "ak", "ym", "yk"))
+        y8 = ws.buf("y8", (R, I_), torch.int8)
         L0 = self.layers[0]
-        P, ns, st = self._gemm(x8, L0.wqkv, (L0.pf_attn,))
+        P, ns, st = self._gemm(x8, L0.wqkv, (L0.pf_attn,), ws=ws, name="P_qkv")
         for li, L in enumerate(self.layers):
             nxt = self.layers[li + 1] if li + 1 < self.n_layers else None
-            attn = self._attend(L, B, 1, P, ns, st, xm, xk, pos, cache, S_past, S, static)
-            Po, nso, sto = self._partials(R, H, nq * hd)
+            attn = self._attend(ws, L, B, 1, P, ns, st, xm, xk, pos, cache, S_past, S, static)
+            Po, nso, sto = self._partials(ws, "P_o", R, H, nq * hd)
             if attn[3] is not None:
                 call("detllm_igemv_merge_ext", L.wo, Po, R, H, nq * hd, nso, sto, attn[0],
                      L.osc_m, L.os_k, L.attn_out_col_k, attn[3], self.n_kv, am, ak, 0,
@@ -555,7 +579,7 @@ class IntQwen3:
                 call("detllm_igemv_merge", L.wo, Po, R, H, nq * hd, nso, sto, *attn[:3],
                      L.osc_m, L.os_k, None, L.attn_out_col_k, am, ak, L.pf_o,
                      L.pf_o.numel() * 8, None, 0)
-            Pg, nsg, stg = self._partials(R, 2 * I_, H)
+            Pg, nsg, stg = self._partials(ws, "P_gu", R, 2 * I_, H)
             call("detllm_igemv_resnormq", L.wgu, Pg, R, 2 * I_, H, nsg, stg, Po, nso, sto, am, ak,
                  L.o_m, L.o_k, 20, hb[cur], kb[cur], hb[1 - cur], kb[1 - cur], L.ms_m, L.ms_k,
                  xm, xk, L.pf_mlp, L.pf_mlp.numel() * 8, None, 0)
@@ -564,7 +588,7 @@ class IntQwen3:
             ksd = self.fused_swiglu_ksplit
             if ksd and I_ % 512 == 0 and I_ <= 3072 and pro_fits(I_, ksd):
                 # the down GEMV computes its SwiGLU operand row itself
-                Pd = torch.empty(ksd, R, H, dtype=torch.int32, device=dev)
+                Pd = ws.buf("P_d", (ksd, R, H), torch.int32)
                 nsd, std = ksd, R * H
                 pf = []
                 for t in pfd:
@@ -575,43 +599,41 @@ class IntQwen3:
             else:
                 call("detllm_swiglu_quant", Pg, nsg, stg, R, I_, xm, xk, L.gate_m, L.gate_k,
                      L.up_m, L.up_k, L.ds_m, L.ds_k, y8, ym, yk, *self._next_gemm(L.wd, R), 0)
-                Pd, nsd, std = self._gemm(y8, L.wd, pfd)
+                Pd, nsd, std = self._gemm(y8, L.wd, pfd, ws=ws, name="P_d")
             if nxt is None:
                 call("detllm_residual_normq", Pd, nsd, std, R, H, ym, yk, L.down_m, L.down_k, 20,
                      hb[cur], kb[cur], None, 0, x8, xm, xk, None, 0, 0, 0, 0)
                 break
             N = nxt.wqkv.shape[0]
-            P, ns, st = self._partials(R, N, H)
+            P, ns, st = self._partials(ws, "P_qkv", R, N, H)
             call("detllm_igemv_resnormq", nxt.wqkv, P, R, N, H, ns, st, Pd, nsd, std, ym, yk,
                  L.down_m, L.down_k, 20, hb[cur], kb[cur], hb[1 - cur], kb[1 - cur], nxt.as_m,
                  nxt.as_k, xm, xk, nxt.pf_attn, nxt.pf_attn.numel() * 8, None, 0)
             cur = 1 - cur
 
-    def _decode_scratch(self, B, S):
+    def _decode_scratch(self, ws: _Workspace, B, S):
         """Global score scratch of the decode attention when the scores of a
         (row, kv-head) do not fit its 48 KiB of LDS."""
         G = self.n_q // self.n_kv
         Spad = (S + 15) // 16 * 16
         if G * Spad * 4 <= 48 * 1024:
             return None
-        return torch.empty(B, self.n_q, Spad, dtype=torch.int32, device=self.device)
+        return ws.buf("scratch", (B, self.n_q, Spad), torch.int32)
 
-    def _attention(self, L, B, T, P, ns, st, xm, xk, pos, cache, S_past, S, static, attn):
-        dev = self.device
+    def _attention(self, ws: _Workspace, L, B, T, P, ns, st, xm, xk, pos, cache, S_past, S, static,
+                   attn):
         nq, nkv, hd, li = self.n_q, self.n_kv, self.hd, L.idx
-        q8 = torch.empty(B, nq, T, hd, dtype=torch.int8, device=dev)
-        tpos = torch.empty(B, nq, T, dtype=I64, device=dev)
+        q8 = ws.buf("q8", (B, nq, T, hd), torch.int8)
+        tpos = ws.buf("tpos", (B, nq, T), I64)
         call("detllm_qkv_epilogue", P, ns, st, B, T, nq, nkv, xm, xk, pos,
-             L.q_m, L.q_k, L.k_m, L.k_k, L.v_m, L.v_k, L.q_norm_m, L.q_norm_k,
-             L.k_norm_m, L.k_norm_k, L.qs_m, L.qs_k, L.kq_m, L.kq_k, L.ks_m, L.ks_k,
-             L.vq_m, L.vq_k, self.rope_cos, self.rope_sin, self.max_pos, q8, tpos, None,
+             *L.epi, q8, tpos, None,
              *cache.layer_args(li), cache.len_idx if static else None,
              0 if static else S_past, L.kq_est, self._err)
-        valid = cache.valid_buf.view(torch.uint8)
+        valid = ws.valid
         if T == 1:
             call("detllm_attn_decode", q8, tpos, *cache.layer_args(li), valid, cache.cap,
                  B, S, nq, nkv, cache.nslots if static else None,
-                 self._decode_scratch(B, S), attn, self._err)
+                 self._decode_scratch(ws, B, S), attn, self._err)
         else:
             call("detllm_attn_prefill", q8, tpos, *cache.layer_args(li), valid, cache.cap,
                  B, T, S_past, nq, nkv, attn)
@@ -631,9 +653,7 @@ class IntQwen3:
         tpos = torch.empty(B, nq, T, dtype=I64, device=dev)
         dbg = torch.empty(B, nq, T, 4, dtype=I64, device=dev)
         call("detllm_qkv_epilogue", P, ns, st, B, T, nq, nkv, xm, xk, pos,
-             L.q_m, L.q_k, L.k_m, L.k_k, L.v_m, L.v_k, L.q_norm_m, L.q_norm_k,
-             L.k_norm_m, L.k_norm_k, L.qs_m, L.qs_k, L.kq_m, L.kq_k, L.ks_m, L.ks_k,
-             L.vq_m, L.vq_k, self.rope_cos, self.rope_sin, self.max_pos, q8, tpos, dbg,
+             *L.epi, q8, tpos, dbg,
              *cache.layer_args(li), None, S_past, L.kq_est, self._err)
         qm, qk = dbg[..., 0:1], dbg[..., 1:2]
         Pfull = P.view(ns, B, T, -1).sum(dim=0, dtype=torch.int32) if ns > 1 else \
@@ -668,13 +688,11 @@ class IntQwen3:
         a = torch.cat(parts, dim=2) if len(parts) > 1 else parts[0]
         attn.copy_(a.permute(0, 2, 1, 3).reshape(B * T, nq * hd))
 
-    def _after_attention(self, L, nxt, B, T, attn, h, k_res, x8, xm, xk):
+    def _after_attention(self, ws: _Workspace, L, nxt, B, T, attn, h, k_res, x8, xm, xk):
         """attn: (context partials, nsplit, split_stride) as _attend returns."""
-        dev = self.device
         R, H, nq, hd, I_ = B * T, self.hidden, self.n_q, self.hd, self.inter
-        a8 = torch.empty(R, nq * hd, dtype=torch.int8, device=dev)
-        am = torch.empty(R, dtype=I64, device=dev)
-        ak = torch.empty(R, dtype=I64, device=dev)
+        a8 = ws.buf("a8", (R, nq * hd), torch.int8)
+        am, ak, ym, yk = (ws.buf(n, (R,), I64) for n in ("am", "ak", "ym", "yk"))
         # decode sizes: the merge and the SwiGLU leave their scale fits to the
         # residual kernel after the next GEMM (same integers)
         dfit = 1 if R <= 64 else 0
@@ -686,16 +704,15 @@ class IntQwen3:
         else:
             call("detllm_merge_rowcol", *attn[:3], R, nq * hd, L.os_m, L.os_k,
                  L.attn_out_col_m, L.attn_out_col_k, a8, am, ak, *self._next_gemm(L.wo, R), dfit)
-        P, ns, st = self._gemm(a8, L.wo, (L.pf_o,))
+        P, ns, st = self._gemm(a8, L.wo, (L.pf_o,), ws=ws, name="P_o")
         call("detllm_residual_normq", P, ns, st, R, H, am, ak, L.o_m, L.o_k, 20, h, k_res,
              L.ms_m, L.ms_k, x8, xm, xk, *self._next_gemm(L.wgu, R), dfit)
-        P, ns, st = self._gemm(x8, L.wgu, (L.pf_mlp,))
-        y8 = torch.empty(R, I_, dtype=torch.int8, device=dev)
-        ym = torch.empty(R, dtype=I64, device=dev)
-        yk = torch.empty(R, dtype=I64, device=dev)
+        P, ns, st = self._gemm(x8, L.wgu, (L.pf_mlp,), ws=ws, name="P_gu")
+        y8 = ws.buf("y8", (R, I_), torch.int8)
         call("detllm_swiglu_quant", P, ns, st, R, I_, xm, xk, L.gate_m, L.gate_k, L.up_m,
              L.up_k, L.ds_m, L.ds_k, y8, ym, yk, *self._next_gemm(L.wd, R), dfit)
-        P, ns, st = self._gemm(y8, L.wd, (L.down_m,) if nxt is None else (L.down_m, nxt.as_m))
+        P, ns, st = self._gemm(y8, L.wd, (L.down_m,) if nxt is None else (L.down_m, nxt.as_m),
+                               ws=ws, name="P_d")
         sm_m, sm_k = (nxt.as_m, nxt.as_k) if nxt is not None else (None, 0)
         call("detllm_residual_normq", P, ns, st, R, H, ym, yk, L.down_m, L.down_k, 20, h, k_res,
              sm_m, sm_k, x8, xm, xk, *self._next_gemm(None if nxt is None else nxt.wqkv, R), dfit)
