@@ -138,6 +138,13 @@ __global__ __launch_bounds__(256) void k_gemm_nt(const int8_t* __restrict__ A,
 // issue overwrites. Tiles are ordered so that each XCD (blocks are dispatched
 // round-robin over the 8 XCDs) owns one contiguous block of the tile grid,
 // keeping its share of A and B in its own L2.
+//
+// KG > 1: KG groups of waves take every KG-th slice of K and their sums meet
+// in LDS at the end. A product of few tiles leaves each SIMD one wave, whose
+// step is a serial chain (wait, barrier, LDS read, dependent MFMAs: about 0.4
+// us per 128-byte slice whatever the tile); groups run such chains side by
+// side and make each KG times shorter. 200 x 1024 with K = 3072: 10.7 us in
+// 128 x 64 tiles, 7.7 in 64 x 32 tiles of four groups; K = 2048: 8.2 -> 6.2.
 // ---------------------------------------------------------------------------
 typedef int v16i __attribute__((ext_vector_type(16)));
 
@@ -163,21 +170,21 @@ __device__ __forceinline__ void g2_tile(int bid, int tiles_m, int tiles_n, int& 
 
 constexpr int G2_BK = 128;
 
-template <int BM, int BN, int S, int WGM, int WGN, int MINB>
-__global__ __launch_bounds__(64 * WGM * WGN, MINB) void k_gemm_nt2(const int8_t* __restrict__ A,
-                                                        const int8_t* __restrict__ B,
-                                                        int32_t* __restrict__ C, int M, int N,
-                                                        int K, i64 sA, i64 sB, i64 sC,
-                                                        int tiles_m, int tiles_n) {
+template <int BM, int BN, int S, int WGM, int WGN, int MINB, int KG = 1>
+__global__ __launch_bounds__(64 * WGM * WGN * KG, MINB) void k_gemm_nt2(
+    const int8_t* __restrict__ A, const int8_t* __restrict__ B, int32_t* __restrict__ C, int M,
+    int N, int K, i64 sA, i64 sB, i64 sC, int tiles_m, int tiles_n) {
   keep_hidden_args();
   constexpr int ROWS = BM + BN;       // 128-byte rows per slice: A rows, then B rows
-  constexpr int NW = WGM * WGN;       // waves, WGM x WGN over the tile
+  constexpr int NW = WGM * WGN;       // waves of a K group, WGM x WGN over the tile
   constexpr int NI = ROWS / 8;        // load instructions per slice (8 rows each)
   static_assert(NI % NW == 0, "loads per wave");
   constexpr int LPW = NI / NW;
-  constexpr int STAGE = ROWS * G2_BK;
+  constexpr int SLICE = ROWS * G2_BK;
+  constexpr int STAGE = SLICE * KG;   // one slice per K group
   constexpr int WA = BM / 32 / WGM, WB = BN / 32 / WGN;  // 32x32 blocks per wave
   static_assert(WA >= 1 && WB >= 1, "wave tile");
+  static_assert((KG - 1) * BM * BN * 4 <= S * STAGE, "the groups' sums fit the ring");
   __shared__ __attribute__((aligned(1024))) int8_t lds[S * STAGE];
 
   const int bz = blockIdx.z;
@@ -186,11 +193,14 @@ __global__ __launch_bounds__(64 * WGM * WGN, MINB) void k_gemm_nt2(const int8_t*
   C += bz * sC;
   int tm, tn;
   g2_tile(blockIdx.x, tiles_m, tiles_n, tm, tn);
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wv = tid >> 6, kg = KG > 1 ? __builtin_amdgcn_readfirstlane(wv / NW) : 0;
+  const int wave = wv - kg * NW;
   const int wm = wave / WGN, wn = wave % WGN;
 
   // this wave's loads: instruction i covers slice rows 8i..8i+7; lane l takes
-  // row 8i + l/8 at physical chunk l%8, i.e. logical chunk (l%8) ^ swz(row)
+  // row 8i + l/8 at physical chunk l%8, i.e. logical chunk (l%8) ^ swz(row).
+  // Group kg takes the slices kg, kg + KG, ...
   const int8_t* src[LPW];
   int dst_off[LPW];
 #pragma unroll
@@ -200,18 +210,18 @@ __global__ __launch_bounds__(64 * WGM * WGN, MINB) void k_gemm_nt2(const int8_t*
     const int lch = (lane & 7) ^ g2_swz(srow);
     if (srow < BM) {
       const int row = min(tm * BM + srow, M - 1);
-      src[j] = A + (i64)row * K + lch * 16;
+      src[j] = A + (i64)row * K + lch * 16 + kg * G2_BK;
     } else {
       const int col = min(tn * BN + (srow - BM), N - 1);
-      src[j] = B + (i64)col * K + lch * 16;
+      src[j] = B + (i64)col * K + lch * 16 + kg * G2_BK;
     }
-    dst_off[j] = __builtin_amdgcn_readfirstlane(ins * 1024);
+    dst_off[j] = __builtin_amdgcn_readfirstlane(kg * SLICE + ins * 1024);
   }
   auto issue = [&](int kt) {
     int8_t* base = lds + (kt % S) * STAGE;
 #pragma unroll
     for (int j = 0; j < LPW; ++j)
-      __builtin_amdgcn_global_load_lds((gbl_ptr_t)(src[j] + (i64)kt * G2_BK),
+      __builtin_amdgcn_global_load_lds((gbl_ptr_t)(src[j] + (i64)kt * (G2_BK * KG)),
                                        (lds_ptr_t)(base + dst_off[j]), 16, 0, 0);
   };
 
@@ -227,20 +237,23 @@ __global__ __launch_bounds__(64 * WGM * WGN, MINB) void k_gemm_nt2(const int8_t*
       for (int r = 0; r < 16; ++r) acc[i][j][r] = 0;
 
   const int nk = K / G2_BK;
+  const int steps = (nk + KG - 1) / KG;      // ring steps of the block
+  const int own = (nk - kg + KG - 1) / KG;   // of them with a slice of this group (steps or one less)
 #pragma unroll
   for (int s = 0; s < S - 1; ++s)
-    if (s < nk) issue(s);
-  for (int kt = 0; kt < nk; ++kt) {
-    // slices issued after kt so far: min(S - 2, nk - 1 - kt)
-    const int after = min(S - 2, nk - 1 - kt);
+    if (s < own) issue(s);
+  for (int kt = 0; kt < steps; ++kt) {
+    // this group's slices issued after kt so far: min(S - 2, own - 1 - kt)
+    const int after = min(S - 2, own - 1 - kt);
     static_assert(S <= 5 && 3 * LPW < 64, "vmcnt range");
     if (after >= 3) wait_vmcnt<3 * LPW>();
     else if (after == 2) wait_vmcnt<2 * LPW>();
     else if (after == 1) wait_vmcnt<LPW>();
     else wait_vmcnt<0>();
     __builtin_amdgcn_s_barrier();
-    if (kt + S - 1 < nk) issue(kt + S - 1);
-    const int8_t* base = lds + (kt % S) * STAGE;
+    if (kt + S - 1 < own) issue(kt + S - 1);
+    if (KG > 1 && kt >= own) continue;  // (the last step may lack this group's slice)
+    const int8_t* base = lds + (kt % S) * STAGE + kg * SLICE;
 #pragma unroll
     for (int s = 0; s < G2_BK / 32; ++s) {
       v4i af[WA], bf[WB];
@@ -259,6 +272,32 @@ __global__ __launch_bounds__(64 * WGM * WGN, MINB) void k_gemm_nt2(const int8_t*
 #pragma unroll
         for (int j = 0; j < WB; ++j) acc[i][j] = mfma32(af[i], bf[j], acc[i][j]);
     }
+  }
+  if constexpr (KG > 1) {
+    // the groups' sums through the ring, group 0 stores
+    __syncthreads();  // every group is done reading it
+    int32_t* part = (int32_t*)lds;
+    constexpr int PER = WA * WB * 16;  // values per lane
+    if (kg > 0) {
+#pragma unroll
+      for (int i = 0; i < WA; ++i)
+#pragma unroll
+        for (int j = 0; j < WB; ++j)
+#pragma unroll
+          for (int r = 0; r < 16; ++r)
+            part[(((kg - 1) * NW + wave) * PER + (i * WB + j) * 16 + r) * 64 + lane] = acc[i][j][r];
+    }
+    __syncthreads();
+    if (kg > 0) return;
+#pragma unroll
+    for (int q = 0; q < KG - 1; ++q)
+#pragma unroll
+      for (int i = 0; i < WA; ++i)
+#pragma unroll
+        for (int j = 0; j < WB; ++j)
+#pragma unroll
+          for (int r = 0; r < 16; ++r)
+            acc[i][j][r] += part[((q * NW + wave) * PER + (i * WB + j) * 16 + r) * 64 + lane];
   }
   // 32x32 result block: lane l, element r -> row 8(r/4) + 4(l/32) + r%4, col l%32
 #pragma unroll
@@ -777,24 +816,37 @@ int detllm_igemm_nt(const int8_t* A, const int8_t* B, int32_t* C, int M, int N, 
   if (K <= 0 || (K % 16) != 0 || K > 131071 || !A || !B || !C) return DI_EINVAL;
   if (batch > 65535) return DI_ERANGE;
   if (M > 64 && K % G2_BK == 0) {
-    // Tile shape by tile count (a sweep of shapes over the four M = 2048
-    // products picked these): 256x256 only for large products (c4 prefill),
-    // 128x192 (two blocks per CU) where it divides N (gate|up), 128x128 (two
-    // per CU) at >= 448 tiles (q|k|v), else 128x64 with a 4-slice ring (o,
-    // down).
+    // Tile shape by tile count, from sweeps of every shape over the model's
+    // four products at 65 to 2048 rows. n = tiles of 128 x 64; us of the taken
+    // shape against 128 x 64 (one block per CU):
+    //   n <= 64: 64 x 32 in four K groups, four times the blocks (o and down
+    //     at 65 to 512 rows: 6.2 / 8.2 and 7.5 / 10.7)
+    //   n <= 128, K >= 2048: 64 x 64 in two K groups (1024 rows: 7.9 / 9.0 and
+    //     9.9 / 11.7); shorter K: 64 x 64 without groups (gate|up at 100 rows
+    //     6.1 / 6.6; in groups 6.3: four steps each, and the sum costs as much)
+    //   n <= 256: 128 x 64
+    //   n <= 512: 64 x 128, two blocks per CU (q|k|v at 1024 rows 9.7 / 11.5)
+    //   more: 128 x 128, two per CU (gate|up at 1024 rows 12.6 / 15.7), and by
+    //     their own counts 128 x 192 (two per CU) where it divides N (gate|up
+    //     at 2048 rows) and 256 x 256 for large products.
     auto tiles = [&](int bm, int bn) { return (i64)((M + bm - 1) / bm) * ((N + bn - 1) / bn) * batch; };
-#define DI_GEMM2(BM, BN, S, WGM, WGN, MINB)                                                      \
+#define DI_GEMM2(BM, BN, S, WGM, WGN, MINB, KG)                                                 \
   do {                                                                                          \
     const int tm_ = (M + BM - 1) / BM, tn_ = (N + BN - 1) / BN;                                 \
     if ((i64)tm_ * tn_ > 0x7fffffff) return DI_ERANGE;                                          \
-    hipLaunchKernelGGL((k_gemm_nt2<BM, BN, S, WGM, WGN, MINB>), dim3(tm_ * tn_, 1, batch),     \
-                       dim3(64 * WGM * WGN), 0, s, A, B, C, M, N, K, (i64)sA, (i64)sB, (i64)sC, \
-                       tm_, tn_);                                                               \
+    hipLaunchKernelGGL((k_gemm_nt2<BM, BN, S, WGM, WGN, MINB, KG>), dim3(tm_ * tn_, 1, batch), \
+                       dim3(64 * WGM * WGN * KG), 0, s, A, B, C, M, N, K, (i64)sA, (i64)sB,     \
+                       (i64)sC, tm_, tn_);                                                      \
   } while (0)
-    if (tiles(256, 256) >= 448) DI_GEMM2(256, 256, 2, 4, 2, 1);
-    else if (N % 192 == 0 && tiles(128, 192) >= 448) DI_GEMM2(128, 192, 2, 2, 2, 2);
-    else if (tiles(128, 128) >= 448) DI_GEMM2(128, 128, 2, 2, 2, 2);
-    else DI_GEMM2(128, 64, 4, 4, 2, 1);
+    const i64 n = tiles(128, 64);
+    if (tiles(256, 256) >= 448) DI_GEMM2(256, 256, 2, 4, 2, 1, 1);
+    else if (N % 192 == 0 && tiles(128, 192) >= 448) DI_GEMM2(128, 192, 2, 2, 2, 2, 1);
+    else if (n > 512) DI_GEMM2(128, 128, 2, 2, 2, 2, 1);
+    else if (n > 256) DI_GEMM2(64, 128, 3, 2, 2, 2, 1);
+    else if (n > 128) DI_GEMM2(128, 64, 4, 4, 2, 1, 1);
+    else if (n <= 64) DI_GEMM2(64, 32, 3, 2, 1, 1, 4);
+    else if (K >= 2048) DI_GEMM2(64, 64, 4, 2, 2, 1, 2);
+    else DI_GEMM2(64, 64, 4, 2, 2, 2, 1);
 #undef DI_GEMM2
     DI_LAUNCH_CHECK();
     return DI_OK;

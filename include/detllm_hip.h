@@ -46,9 +46,9 @@ extern "C" {
 /* int_gemm(a, b, backend) — src/detllm/backends.py:88-135 (batched form
  * :127-134). C[b] = A[b] . B[b]^T: A [batch][M][K], B [batch][N][K] (the
  * artifact's [K][N] w8t transposed), C [batch][M][N] int32; batch strides in
- * elements. K % 16 == 0, K <= 131071. i8 MFMA: 32x32x32 tiles of 256x256,
- * 128x192, 128x128 or 128x64 elements per block by tile count when K % 128
- * == 0 (a direct-to-LDS operand ring), else 128x128 blocks of 16x16x64. */
+ * elements. K % 16 == 0, K <= 131071. i8 MFMA: 32x32x32 tiles of 256x256 down
+ * to 64x32 elements per block by tile count when K % 128 == 0 (a direct-to-LDS
+ * operand ring), else 128x128 blocks of 16x16x64. */
 int detllm_igemm_nt(const int8_t* A, const int8_t* B, int32_t* C, int M, int N, int K,
                     int batch, int64_t sA, int64_t sB, int64_t sC, hipStream_t s);
 
