@@ -58,6 +58,7 @@ struct PrefillArgs {
 constexpr int PF_KBYTES = 128 * 128;      // K tile: 128 slot rows of 128 B
 constexpr int PF_VBYTES = 128 * 128;      // V^T tile: 128 dim rows of 128 B
 constexpr int PF_RING = 64 * 1024;        // 4 K stages, or 2 K+V stages
+constexpr int PF_RESIDENT = PF_RING / (PF_KBYTES + PF_VBYTES);  // pages whose K and V fit the ring
 constexpr int PF_CSUM = 128 * 4;          // column sums of V (int32 per dim)
 constexpr uint32_t PF_SMALL_T = 1u << 23;  // estimated DI-Exp below this tpos
 constexpr i64 PF_SMALL_DEN = (i64)1 << 34;  // estimated p below this den
@@ -146,7 +147,52 @@ __global__ __launch_bounds__(256, 2) void k_attn_prefill(PrefillArgs a) {
   const int ntiles = (kend + 63) / 64;
   const uint8_t* vrow = a.valid + (i64)b * a.valid_stride;
   const int ntiles2 = (ntiles + 1) / 2;  // 128-slot tiles = pages
-  for (int i = tid; i < ntiles2; i += 256) pages[i] = a.kv.page(b, (i64)i * DI_PAGE);
+
+  // Key tiles of 128 slots reach LDS by direct-to-LDS loads; each tile is
+  // processed as two 64-slot halves (the 64-slot tiles `it` of the masks). K:
+  // instruction j of wave w covers tile rows 8(4w + j) .. +7, lane l row
+  // 8(4w + j) + l/8 at physical chunk l % 8; V^T likewise with dims for rows.
+  // A tile is one page; the buffer resources span that page's (kv head) part,
+  // 16 KB of K and of V^T. A page that is not mapped gets a zero-length
+  // resource, so its loads read 0. Slots past the scanned range in a mapped
+  // page read whatever the page holds; such slots are never visible (p = 0:
+  // their hi byte -64 and the +64 column-sum term cancel).
+  int koffl[4], voffl[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int row = (wave * 4 + j) * 8 + (lane >> 3);
+    koffl[j] = row * 128 + ((lane & 7) ^ pf_kswz(row)) * 16;
+    voffl[j] = row * DI_PAGE + ((lane & 7) ^ pf_vswz(row)) * 16;
+  }
+  auto issue = [&](int page, int8_t* st, bool with_v) {
+    const int pg = __builtin_amdgcn_readfirstlane(page);
+    const int pgc = pg < 0 ? 0 : pg;
+    const int nrec = pg < 0 ? 0 : DI_PAGE * 128;
+    const __amdgpu_buffer_rsrc_t krs = __builtin_amdgcn_make_buffer_rsrc(
+        (void*)a.kv.krow(pgc, kvh, 0), (short)0, nrec, 0x00020000);
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(krs, (lds_ptr_t)(st + (wave * 4 + j) * 1024), 16,
+                                               koffl[j], 0, 0, 0);
+    if (with_v) {
+      const __amdgpu_buffer_rsrc_t vrs = __builtin_amdgcn_make_buffer_rsrc(
+          (void*)a.kv.vchan(pgc, kvh, 0), (short)0, nrec, 0x00020000);
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(
+            vrs, (lds_ptr_t)(st + PF_KBYTES + (wave * 4 + j) * 1024), 16, voffl[j], 0, 0, 0);
+    }
+  };
+  // A block of few pages keeps all of K and V in the ring for its three
+  // passes: one memory round trip, beside the mask's, and no barrier per tile
+  // (a round trip of each pass's loads is most of a short prompt's launch).
+  const bool resident = ntiles2 <= PF_RESIDENT;
+  if (resident) {
+    for (int i = 0; i < ntiles2; ++i)
+      issue(a.kv.page(b, (i64)i * DI_PAGE), ring + i * (PF_KBYTES + PF_VBYTES), true);
+  } else {
+    for (int i = tid; i < ntiles2; i += 256) pages[i] = a.kv.page(b, (i64)i * DI_PAGE);
+  }
 
   // validity bitmask of every key tile (bit s - 64 i of tile i: slot s < S
   // and valid), made once and read by all three passes for the tiles that
@@ -169,46 +215,12 @@ __global__ __launch_bounds__(256, 2) void k_attn_prefill(PrefillArgs a) {
     }
   }
   if (lane == 0) csum_lds[wave] = nf;  // the column-sum area is free until the end
+  wait_vmcnt<0>();  // query operands in registers before the ring's loads count; resident tiles here
   __syncthreads();
   const int nfull = min(min(csum_lds[0], csum_lds[1]), min(csum_lds[2], csum_lds[3]));
-  wait_vmcnt<0>();  // query operands in registers before the ring's loads count
 
-  // Key tiles of 128 slots stream into an LDS ring with direct-to-LDS loads,
-  // issued STAGES - 1 tiles ahead; each tile is processed as two 64-slot
-  // halves (the 64-slot tiles `it` of the masks) between one barrier and the
-  // next. K: instruction j of wave w covers tile rows 8(4w + j) .. +7, lane l
-  // row 8(4w + j) + l/8 at physical chunk l % 8; V^T likewise with dims for
-  // rows. A tile is one page; the buffer resources span that page's
-  // (kv head) part, 16 KB of K and of V^T. A page that is not mapped gets a
-  // zero-length resource, so its loads read 0. Slots past the scanned range
-  // in a mapped page read whatever the page holds; such slots are never
-  // visible (p = 0: their hi byte -64 and the +64 column-sum term cancel).
-  int koffl[4], voffl[4];
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const int row = (wave * 4 + j) * 8 + (lane >> 3);
-    koffl[j] = row * 128 + ((lane & 7) ^ pf_kswz(row)) * 16;
-    voffl[j] = row * DI_PAGE + ((lane & 7) ^ pf_vswz(row)) * 16;
-  }
-  auto issue = [&](int tile, int8_t* st, bool with_v) {
-    const int pg = __builtin_amdgcn_readfirstlane(pages[tile]);
-    const int pgc = pg < 0 ? 0 : pg;
-    const int nrec = pg < 0 ? 0 : DI_PAGE * 128;
-    const __amdgpu_buffer_rsrc_t krs = __builtin_amdgcn_make_buffer_rsrc(
-        (void*)a.kv.krow(pgc, kvh, 0), (short)0, nrec, 0x00020000);
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(krs, (lds_ptr_t)(st + (wave * 4 + j) * 1024), 16,
-                                               koffl[j], 0, 0, 0);
-    if (with_v) {
-      const __amdgpu_buffer_rsrc_t vrs = __builtin_amdgcn_make_buffer_rsrc(
-          (void*)a.kv.vchan(pgc, kvh, 0), (short)0, nrec, 0x00020000);
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(
-            vrs, (lds_ptr_t)(st + PF_KBYTES + (wave * 4 + j) * 1024), 16, voffl[j], 0, 0, 0);
-    }
-  };
+  // More pages stream through the ring, issued STAGES - 1 tiles ahead, one
+  // barrier per tile.
   // one pass over the key tiles; body(it2, stage) runs with tile it2 in LDS.
   // Each wave waits for its own loads of the tile (vmcnt: loads complete in
   // order), then one barrier publishes every wave's part and frees the
@@ -219,17 +231,21 @@ __global__ __launch_bounds__(256, 2) void k_attn_prefill(PrefillArgs a) {
     constexpr int ST = PF_RING / STAGE;
     constexpr int LPT = KV ? 8 : 4;  // loads per tile per wave
     static_assert(ST >= 2 && ST <= 4 && 2 * LPT < 64, "ring stages");
+    if (resident) {
+      for (int it2 = 0; it2 < ntiles2; ++it2) body(it2, ring + it2 * (PF_KBYTES + PF_VBYTES));
+      return;
+    }
     __builtin_amdgcn_s_barrier();  // the previous pass is done with the ring
 #pragma unroll
     for (int s = 0; s < ST - 1; ++s)
-      if (s < ntiles2) issue(s, ring + s * STAGE, KV);
+      if (s < ntiles2) issue(pages[s], ring + s * STAGE, KV);
     for (int it2 = 0; it2 < ntiles2; ++it2) {
       const int after = min(ST - 2, ntiles2 - 1 - it2);  // tiles issued after it2
       if (after >= 2) wait_vmcnt<2 * LPT>();
       else if (after == 1) wait_vmcnt<LPT>();
       else wait_vmcnt<0>();
       __builtin_amdgcn_s_barrier();
-      if (it2 + ST - 1 < ntiles2) issue(it2 + ST - 1, ring + ((it2 + ST - 1) % ST) * STAGE, KV);
+      if (it2 + ST - 1 < ntiles2) issue(pages[it2 + ST - 1], ring + ((it2 + ST - 1) % ST) * STAGE, KV);
       body(it2, ring + (it2 % ST) * STAGE);
     }
   };

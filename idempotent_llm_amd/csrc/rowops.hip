@@ -1885,14 +1885,16 @@ void launch_pro(const ProGemv& g, int ni, int ksplit, const ResNormArgs& ra, con
   } while (0)
 
 // The wave-per-row launch of a prefill-sized residual / norm-quant call
-// (R > 64 rows of C = 512 or 1024 columns); false: the caller launches the
-// block-per-row kernel.
+// (C = 512 or 1024 columns); false: the caller launches the block-per-row
+// kernel. A wave per row has no barriers, but its chain over 16 columns per
+// lane is long; up to 640 rows a block per row (four columns per lane) fits
+// the chip two or three blocks per CU and is done sooner: residual rows 320 /
+// 512 / 700 / 1024 / 2048 take 7.3 / 7.6 / 8.8 / 10.1 / 14.4 us as blocks, 8.6
+// / 8.8 / 9.1 / 9.3 / 12.5 as waves.
+constexpr int ROWS_WAVE_MIN = 641;
 template <int MODE>
 static bool rows_wave_launch(int R, int C, hipStream_t s, ResNormArgs& a) {
-#ifdef ROWS_BLOCK
-  return false;
-#endif
-  if (R <= 64 || (C != 512 && C != 1024)) return false;
+  if (R < ROWS_WAVE_MIN || (C != 512 && C != 1024)) return false;
   a.nt = 64;
   const dim3 grid((unsigned)((R + 3) / 4));
   if (C == 1024) hipLaunchKernelGGL((k_residual_normq_w<16, MODE>), grid, dim3(256), 0, s, a, R);

@@ -656,3 +656,28 @@ def test_qkv_epilogue_rows_per_lane(variant, B, T, slot):
         np.testing.assert_array_equal(v[:, :, slot:].cpu().numpy(), want_v)
         assert torch.equal(k[:, :, :slot].cpu(), k0[:, :, :slot])   # earlier slots untouched
         assert torch.equal(v[:, :, :slot].cpu(), v0.transpose(2, 3)[:, :, :slot])
+
+
+@pytest.mark.parametrize("T,S_past", [(128, 0), (1, 128), (129, 0), (100, 156), (257, 0),
+                                      (65, 192), (300, 84)])
+def test_prefill_attention_resident_pages(T, S_past):
+    """Blocks whose K and V stay in LDS (at most two pages of keys) next to
+    blocks of the same launch that stream them: one slot to each side of a
+    page and of the two-page limit, with a page in the middle not mapped."""
+    from idempotent_llm_amd._lib import call
+    print(f"[prefill resident pages T={T} S_past={S_past}]", flush=True)
+    B, n_q, n_kv, S = 2, 4, 2, S_past + T
+    cap = -(-S // 128) * 128
+    q8, kc, vc, valid, sm, sk, tpos = _prefill_case(B, n_q, n_kv, T, S_past, cap, S, 29, 34)
+    if cap > 128:
+        valid[1, 0:128] = False          # row 1: page 0 is not mapped
+    want = _prefill_oracle(q8, kc, vc, valid, sm, sk, S_past)
+    d = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()
+    out = torch.full((B, T, n_q * 128), -7, dtype=I64, device="cuda")
+    kp, vp, table, width, vmask = paged(kc, vc, valid, seed=S)
+    if cap > 128:
+        table[1, 0] = -1
+    call("detllm_attn_prefill", d(q8), d(tpos[..., 0]), kp, vp, table, width,
+         vmask.view(torch.uint8), width * 128, B, T, S_past, n_q, n_kv, out)
+    bad = np.argwhere(out.cpu().numpy() != want)
+    assert bad.size == 0, f"{len(bad)} mismatches, first at {bad[0].tolist()}"
