@@ -31,6 +31,7 @@ SIGNATURES = {
     "detllm_igemv_plan": [I, I, I, P],
     "detllm_attn_split_plan": [I, I, I, I, P, P],
     "detllm_transpose_i8": [P, P, I, I, I, L, L, S],
+    "detllm_pack_nt": [P, P, P, P, I, I, I, I, I, S],
     "detllm_greedy_pick": [P, P, I, I, I, P, P, P, S],
     "detllm_greedy_pick_noalloc": [P, P, I, I, P, S],
     "detllm_logits_digest": [P, I, I, P, S],

@@ -17,9 +17,9 @@
 // in element r of lane l.
 //
 // Kernels:
-//   k_gemm_nt2  — M > 64, K % 128 == 0 (prefill): 32x32x32 MFMA, direct-to-LDS
+//   k_gemm_nt2  — K % 128 == 0 (prefill, int_gemm): 32x32x32 MFMA, direct-to-LDS
 //                 operand ring with swizzled rows, XCD-blocked tile order.
-//   k_gemm_nt   — other M > 64 shapes: 128x128x64 block tiles, 4 waves of
+//   k_gemm_nt   — other K: 128x128x64 block tiles, 4 waves of
 //                 64x64, LDS double buffer.
 //   k_gemv_nt   — M <= 64 (decode): a wave owns 16 output columns and a
 //                 K range; weight fragments stream straight from HBM into
@@ -119,7 +119,7 @@ __global__ __launch_bounds__(256) void k_gemm_nt(const int8_t* __restrict__ A,
 }
 
 // ---------------------------------------------------------------------------
-// k_gemm_nt2 — the prefill GEMM (M > 64, K % 128 == 0), on
+// k_gemm_nt2 — the prefill GEMM (K % 128 == 0), on
 // v_mfma_i32_32x32x32_i8: both i8 forms run at the same rate on gfx950
 // (measured, about 4.4 POP/s), but a 32x32x32 tile needs half the operand
 // bytes per multiply-add of a 16x16x64 one, so half the LDS reads.
@@ -619,6 +619,77 @@ __global__ void k_transpose_i8(const int8_t* __restrict__ src, int8_t* __restric
   }
 }
 
+// int_gemm's operands in the products' layout, one launch: bt [batch][N][Kp]
+// = b^T of b [batch][K][N] and, where K is padded, ap [batch][M][Kp] = a
+// [batch][M][K], zeros in the columns K .. Kp (exact in an integer product).
+// Blocks 0 .. tk * tn - 1 of a batch index turn 128 x 64 tiles of b (128
+// output bytes per row: whole lines), the others copy 4096 bytes of ap each.
+// 16-byte loads at any alignment (rows of any length), 4 x 4 bytes turned in
+// registers; bound by latency at these sizes: b of 1000 x 1500 with a of 777
+// rows PACK_US.
+typedef int v4i_u __attribute__((ext_vector_type(4), aligned(1)));
+constexpr int PK_K = 128, PK_N = 64, PK_LD = 17;  // LDS row: 16 words of columns, 1 of padding
+
+__global__ __launch_bounds__(256) void k_pack_nt(const int8_t* __restrict__ a,
+                                                 int8_t* __restrict__ ap,
+                                                 const int8_t* __restrict__ b,
+                                                 int8_t* __restrict__ bt, int M, int N, int K,
+                                                 int Kp, int tk, int tn) {
+  keep_hidden_args();
+  __shared__ uint32_t tile[PK_K * PK_LD];
+  const int tid = threadIdx.x;
+  const i64 z = blockIdx.y;
+  // 16 bytes at p of which the first n are in the operand (n <= 0: none)
+  auto load16 = [](const int8_t* p, int n) -> v4i {
+    if (n >= 16) return *(const v4i_u*)p;
+    uint32_t w[4] = {0, 0, 0, 0};
+    for (int i = 0; i < n; ++i) w[i >> 2] |= (uint32_t)(uint8_t)p[i] << (8 * (i & 3));
+    return v4i{(int)w[0], (int)w[1], (int)w[2], (int)w[3]};
+  };
+  if ((int)blockIdx.x >= tk * tn) {
+    const int kc = Kp >> 4;
+    const i64 i = (i64)(blockIdx.x - tk * tn) * 256 + tid;
+    if (i >= (i64)M * kc) return;
+    const i64 r = i / kc;
+    const int k = (int)(i - r * kc) * 16;
+    *(v4i*)(ap + (z * M + r) * Kp + k) = load16(a + (z * M + r) * K + k, K - k);
+    return;
+  }
+  const int k0 = (int)blockIdx.x / tn * PK_K, n0 = (int)blockIdx.x % tn * PK_N;
+  b += z * (i64)K * N;
+  bt += z * (i64)N * Kp;
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    const int kr = (tid >> 2) + 64 * q, c = (tid & 3) * 16;
+    const v4i v = load16(b + (i64)(k0 + kr) * N + n0 + c, k0 + kr < K ? N - n0 - c : 0);
+#pragma unroll
+    for (int w = 0; w < 4; ++w) tile[kr * PK_LD + (c >> 2) + w] = (uint32_t)v[w];
+  }
+  __syncthreads();
+  const int kq = tid & 31;
+  if (k0 + 4 * kq >= Kp) return;
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    const int c = (tid >> 5) + 8 * q;  // word column: output rows n0 + 4 c .. + 3
+    uint32_t r[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) r[j] = tile[(4 * kq + j) * PK_LD + c];
+    const uint32_t lo01 = __builtin_amdgcn_perm(r[1], r[0], 0x05010400u);
+    const uint32_t lo23 = __builtin_amdgcn_perm(r[3], r[2], 0x05010400u);
+    const uint32_t hi01 = __builtin_amdgcn_perm(r[1], r[0], 0x07030602u);
+    const uint32_t hi23 = __builtin_amdgcn_perm(r[3], r[2], 0x07030602u);
+    const uint32_t o[4] = {__builtin_amdgcn_perm(lo23, lo01, 0x05040100u),
+                           __builtin_amdgcn_perm(lo23, lo01, 0x07060302u),
+                           __builtin_amdgcn_perm(hi23, hi01, 0x05040100u),
+                           __builtin_amdgcn_perm(hi23, hi01, 0x07060302u)};
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int n = n0 + 4 * c + j;
+      if (n < N) *(uint32_t*)(bt + (i64)n * Kp + k0 + 4 * kq) = o[j];
+    }
+  }
+}
+
 struct Best {
   i64 v;
   i64 i;
@@ -815,7 +886,7 @@ int detllm_igemm_nt(const int8_t* A, const int8_t* B, int32_t* C, int M, int N, 
   if (M <= 0 || N <= 0 || batch <= 0) return DI_OK;
   if (K <= 0 || (K % 16) != 0 || K > 131071 || !A || !B || !C) return DI_EINVAL;
   if (batch > 65535) return DI_ERANGE;
-  if (M > 64 && K % G2_BK == 0) {
+  if (K % G2_BK == 0) {  // (M <= 64: batched products, one matrix of few rows takes the skinny kernels)
     // Tile shape by tile count, from sweeps of every shape over the model's
     // four products at 65 to 2048 rows. n = tiles of 128 x 64; us of the taken
     // shape against 128 x 64 (one block per CU):
@@ -912,6 +983,23 @@ int detllm_transpose_i8(const int8_t* src, int8_t* dst, int R, int Cc, int batch
   if (!src || !dst || batch > 65535 || (R + 63) / 64 > 65535) return DI_EINVAL;
   hipLaunchKernelGGL(k_transpose_i8, dim3((Cc + 63) / 64, (R + 63) / 64, batch), dim3(256), 0, s,
                      src, dst, R, Cc, (i64)sS, (i64)sD);
+  DI_LAUNCH_CHECK();
+  return DI_OK;
+}
+
+// int_gemm's operands in the layout of the products above (k_pack_nt); ap
+// null: a is used as it is (K == Kp).
+int detllm_pack_nt(const int8_t* a, int8_t* ap, const int8_t* b, int8_t* bt, int M, int N, int K,
+                   int Kp, int batch, hipStream_t s) {
+  if (N <= 0 || batch <= 0) return DI_OK;
+  if (M < 0 || K < 0 || Kp < 16 || Kp % 16 || Kp < K || Kp > (1 << 24) || batch > 65535 ||
+      (K > 0 && !b) || !bt || ((uintptr_t)bt & 15) || (ap && ((M > 0 && K > 0 && !a) || ((uintptr_t)ap & 15))))
+    return DI_EINVAL;
+  const int tk = (Kp + PK_K - 1) / PK_K, tn = (N + PK_N - 1) / PK_N;
+  const i64 blocks = (i64)tk * tn + (ap ? ((i64)M * (Kp / 16) + 255) / 256 : 0);
+  if (blocks > 0x7fffffff) return DI_ERANGE;
+  hipLaunchKernelGGL(k_pack_nt, dim3((unsigned)blocks, batch), dim3(256), 0, s, a, ap, b, bt, M, N,
+                     K, Kp, tk, tn);
   DI_LAUNCH_CHECK();
   return DI_OK;
 }

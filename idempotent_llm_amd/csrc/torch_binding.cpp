@@ -123,7 +123,7 @@ struct Bind<F> {
 #define DI_ENTRY(NAME) Bind<&NAME>::entry(#NAME)
 const Entry ENTRIES[] = {
     DI_ENTRY(detllm_igemm_nt), DI_ENTRY(detllm_igemv_nt), DI_ENTRY(detllm_igemv_nt_pf),
-    DI_ENTRY(detllm_igemv_plan), DI_ENTRY(detllm_attn_split_plan), DI_ENTRY(detllm_transpose_i8),
+    DI_ENTRY(detllm_igemv_plan), DI_ENTRY(detllm_attn_split_plan), DI_ENTRY(detllm_transpose_i8), DI_ENTRY(detllm_pack_nt),
     DI_ENTRY(detllm_greedy_pick), DI_ENTRY(detllm_greedy_pick_noalloc),
     DI_ENTRY(detllm_logits_digest), DI_ENTRY(detllm_embed_normq), DI_ENTRY(detllm_residual_normq),
     DI_ENTRY(detllm_norm_quant), DI_ENTRY(detllm_attn_decode_split),
@@ -233,24 +233,6 @@ T3 rows_out(int64_t R, int64_t C, const Tensor& like) {
   return {empty({R, C}, at::kChar, like), empty({R}, at::kLong, like), empty({R}, at::kLong, like)};
 }
 
-Tensor transpose_i8(const Tensor& b, int64_t batch) {  // [batch, K, N] -> [batch, N, K]
-  const int64_t K = b.size(-2), N = b.size(-1);
-  const Tensor src = b.contiguous();
-  Tensor dst = empty({batch, N, K}, at::kChar, b);
-  DI_RUN(detllm_transpose_i8, ptr<int8_t>(src), ptr<int8_t>(dst), (int)K, (int)N, (int)batch, K * N,
-         K * N);
-  return dst;
-}
-Tensor pad_k(const Tensor& x, int64_t Kp) {
-  const int64_t K = x.size(-1);
-  if (K == Kp) return x.contiguous();
-  auto shape = x.sizes().vec();
-  shape.back() = Kp;
-  Tensor out = at::zeros(shape, x.options());
-  out.narrow(-1, 0, K).copy_(x);
-  return out;
-}
-
 Tensor op_int_gemm(const Tensor& a, const Tensor& b) {
   if (b.dim() == 2 && a.dim() > 2) {
     auto lead = a.sizes().vec();
@@ -261,12 +243,22 @@ Tensor op_int_gemm(const Tensor& a, const Tensor& b) {
   auto shape = a.sizes().vec();
   shape.back() = N;
   if (M == 0 || N == 0) return at::zeros(shape, a.options().dtype(at::kInt));
-  const int64_t Kp = std::max<int64_t>(16, (K + 15) / 16 * 16);
+  // few rows of one matrix take the skinny kernels (K in steps of 16), the
+  // rest the tiled one, at its best in whole 128-byte slices of K
+  const bool skinny = a.dim() == 2 && M <= 64;
+  const int64_t step = skinny ? 16 : 128;
+  const int64_t Kp = std::max(step, (K + step - 1) / step * step);
   int64_t batch = 1;
   for (int64_t i = 0; i < a.dim() - 2; ++i) batch *= a.size(i);
-  const Tensor bt = pad_k(transpose_i8(b, batch), Kp), ap = pad_k(a, Kp);
+  const Tensor ac = a.contiguous(), bc = b.contiguous();
+  // (the products load 16 bytes at a time)
+  const bool as_is = K == Kp && (reinterpret_cast<uintptr_t>(ac.data_ptr()) & 15) == 0;
+  const Tensor bt = empty({batch, N, Kp}, at::kChar, a);
+  const Tensor ap = as_is ? ac : empty({batch, M, Kp}, at::kChar, a);
+  DI_RUN(detllm_pack_nt, ptr<int8_t>(ac), as_is ? nullptr : ptr<int8_t>(ap), ptr<int8_t>(bc),
+         ptr<int8_t>(bt), (int)M, (int)N, (int)K, (int)Kp, (int)batch);
   Tensor out = empty(shape, at::kInt, a);
-  if (a.dim() == 2 && M <= 64)
+  if (skinny)
     DI_RUN(detllm_igemv_nt, ptr<int8_t>(ap), ptr<int8_t>(bt), ptr<int32_t>(out), (int)M, (int)N,
            (int)Kp, 1, M * N);
   else

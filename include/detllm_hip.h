@@ -80,6 +80,14 @@ int detllm_igemv_plan(int M, int N, int K, int* ksplit);
 int detllm_transpose_i8(const int8_t* src, int8_t* dst, int R, int C, int batch,
                         int64_t sS, int64_t sD, hipStream_t s);
 
+/* int_gemm's operands (backends.py:88-135) in the layout of the products
+ * above, one launch: bt [batch][N][Kp] the transpose of b [batch][K][N] and,
+ * with ap non-null, ap [batch][M][Kp] = a [batch][M][K]; columns K .. Kp - 1
+ * are zero. Kp a multiple of 16 (128 for detllm_igemm_nt's wide tiles), ap and
+ * bt 16-byte aligned, a and b at any alignment. */
+int detllm_pack_nt(const int8_t* a, int8_t* ap, const int8_t* b, int8_t* bt, int M, int N, int K,
+                   int Kp, int batch, hipStream_t s);
+
 /* IntQwen3.greedy_pick — src/detllm/model.py:482-490: out[r] = lowest v
  * maximising logits[r][v] * head_m[v] (int64). pv/pi: R * ceil(V/chunk)
  * int64 scratch each. */

@@ -71,3 +71,35 @@ def test_tile_rules_batched():
         for b in range(batch):
             assert torch.equal(out[b, :M], _want(a[b, :M], w[b, :N])), b
         assert (out[:, M:] == 7).all()
+
+
+@pytest.mark.parametrize("M,K,N", [(1, 1, 1), (3, 17, 5), (64, 100, 70), (65, 1, 3), (65, 127, 64),
+                                   (66, 128, 65), (70, 129, 1), (130, 1000, 129), (200, 48, 63),
+                                   (64, 128, 4097), (1000, 333, 257)])
+@pytest.mark.parametrize("form", ["plain", "offset", "strided"])
+def test_int_gemm_operands(M, K, N, form):
+    """backends.int_gemm on operands of every row length, at odd storage
+    offsets and non-contiguous (both transposed views)."""
+    from idempotent_llm_amd.backends import int_gemm
+    print(f"[int_gemm operands M={M} K={K} N={N} {form}]", flush=True)
+    if form == "strided":
+        a, b = _i8(M, K + 3, M).t()[:, :K], _i8(N, N, K + 1).t()[:K]
+    else:
+        off = 3 if form == "offset" else 0
+        a = _i8(M, M * K + off + 8)[off:off + M * K].view(M, K)
+        b = _i8(N, K * N + off + 8)[off:off + K * N].view(K, N)
+    assert torch.equal(int_gemm(a, b, "rocm"), (a.double() @ b.double()).to(torch.int32))
+
+
+@pytest.mark.parametrize("lead,M,K,N", [((3,), 1, 128, 200), ((2, 4), 33, 128, 65),
+                                        ((5,), 64, 60, 31), ((16,), 200, 128, 400), ((0,), 4, 8, 4),
+                                        ((2,), 7, 0, 3)])
+def test_int_gemm_batched(lead, M, K, N):
+    """Batched products, few rows each on the tiled kernel; an empty batch
+    and an empty K."""
+    from idempotent_llm_amd.backends import int_gemm
+    print(f"[int_gemm batched {lead} M={M} K={K} N={N}]", flush=True)
+    a = torch.randint(-128, 128, (*lead, M, K), dtype=torch.int8, device="cuda")
+    b = torch.randint(-128, 128, (*lead, K, N), dtype=torch.int8, device="cuda")
+    want = torch.matmul(a.cpu().double(), b.cpu().double()).to(torch.int32)
+    assert torch.equal(int_gemm(a, b, "rocm").cpu(), want)
