@@ -39,6 +39,7 @@ SIGNATURES = {
     "detllm_residual_normq": [P, I, L, I, I, P, P, P, L, I, P, P, P, L, P, P, P, P, I, I, I, I, S],
     "detllm_norm_quant": [P, I, I, P, L, P, P, P, S],
     "detllm_attn_decode_split": [P, P, P, P, P, I, P, L, I, I, I, I, P, I, P, P, P, P, S],
+    "detllm_attn_decode_split_sum": [P, P, P, P, P, I, P, L, I, I, I, I, P, I, P, P, P, P, S],
     "detllm_igemv_resnormq": [P, P, I, I, I, I, L, P, I, L, P, P, P, L, I, P, P, P, P, P, L, P,
                               P, P, L, P, L, S],
     "detllm_igemv_merge": [P, P, I, I, I, I, L, P, I, L, P, L, P, L, P, P, P, L, P, L, S],

@@ -554,10 +554,11 @@ __device__ __forceinline__ void p_frags(const int32_t* pp, v4i& ahi, v4i& alo) {
 // (grp, l16), element r holds head 4 grp + r, channel 16 (NB wave + nb) + l16;
 // the colsum of that channel sits in row G (lane 16 (G / 4) + l16, element
 // G % 4). out_heads: the block's first head row of [.][128] int64.
-// each(nb, r, value) sees every stored value.
+// each(nb, r, value) sees every stored value. add: the values are added to
+// out_heads (several blocks share it) instead of stored.
 template <int G, int NB = 2, class Each>
 __device__ __forceinline__ void store_pv(const v4i (&chi)[NB], const v4i (&clo)[NB],
-                                         int64_t* out_heads, Each&& each) {
+                                         int64_t* out_heads, Each&& each, bool add = false) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, l16 = lane & 15, grp = lane >> 4;
 #pragma unroll
   for (int nb = 0; nb < NB; ++nb) {
@@ -569,7 +570,8 @@ __device__ __forceinline__ void store_pv(const v4i (&chi)[NB], const v4i (&clo)[
       const int hh = grp * 4 + r;
       if (hh < G) {
         const i64 o = ((i64)chi[nb][r] + 64 * (i64)cs) * 128 + (i64)clo[nb][r];
-        out_heads[hh * 128 + d] = o;
+        if (add) atomicAdd((unsigned long long*)&out_heads[hh * 128 + d], (unsigned long long)o);
+        else out_heads[hh * 128 + d] = o;
         each(nb, r, o);
       }
     }
@@ -577,8 +579,8 @@ __device__ __forceinline__ void store_pv(const v4i (&chi)[NB], const v4i (&clo)[
 }
 template <int G, int NB = 2>
 __device__ __forceinline__ void store_pv(const v4i (&chi)[NB], const v4i (&clo)[NB],
-                                         int64_t* out_heads) {
-  store_pv<G, NB>(chi, clo, out_heads, [](int, int, i64) {});
+                                         int64_t* out_heads, bool add = false) {
+  store_pv<G, NB>(chi, clo, out_heads, [](int, int, i64) {}, add);
 }
 
 // The slots a decode block scans: a.S, bounded by the device count when one
@@ -1166,6 +1168,7 @@ __global__ __launch_bounds__(QAD_WAVES * 64) void k_qkv_attn_decode(DecodeArgs a
 
 constexpr int SPLIT_MAX_CHUNK = 4096;                  // slots per chunk
 constexpr int SPLIT_MAX_PAGES = SPLIT_MAX_CHUNK / DI_PAGE;
+constexpr int SPLIT_DL = 4;  // 16-byte loads of scores in flight per thread and head
 
 struct SplitArgs {
   DecodeArgs d;     // scratch: scores [B][n_q][spad]; out: partials [ns][B][n_q * 128]
@@ -1173,6 +1176,9 @@ struct SplitArgs {
   int chunk, ns;
   i64 spad;         // row stride of the scores (>= S)
   i64 out_stride;   // elements between partials (B * n_q * 128)
+  // out is one [B][n_q * 128] context: zeroed by the scores launch, every
+  // chunk's partial added to it (integer adds: any order gives the same sum)
+  int add;
 };
 
 template <int G>
@@ -1184,24 +1190,30 @@ __global__ __launch_bounds__(256) void k_attn_split_scores(SplitArgs sa) {
   BlockRedT<4> red{red_buf, 0, 256};
   const int kvh = blockIdx.x, b = blockIdx.y, c = blockIdx.z;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, l16 = lane & 15, grp = lane >> 4;
-  bool over;
-  const int S = scanned_slots(a, a.tpos, &over);
-  report_slots(a, over, kvh == 0 && c == 0);  // every later load depends on S anyway
-  const int lo = c * sa.chunk, hi = ::min(lo + sa.chunk, S);
+  const int lo = c * sa.chunk;
   const i64 q0 = (i64)b * a.n_q + kvh * G;
-  int32_t* cm = sa.cmax + q0 * sa.ns + c;  // head hh at cm[hh * ns]
-  if (lo >= hi) {  // block-uniform: a chunk past the scanned slots
-    if (tid < G) cm[tid * sa.ns] = SCORE_MASKED;
-    return;
-  }
-  const int npg = (hi - lo + DI_PAGE - 1) / DI_PAGE;
-  if (tid < npg) pg_lds[tid] = a.kv.page(b, (i64)lo + (i64)tid * DI_PAGE);
+  // the chunk's pages (below the launch's bound a.S) and the queries load
+  // beside the device's slot count, not after it
+  const int npg = (::min(sa.chunk, a.S - lo) + DI_PAGE - 1) / DI_PAGE;
+  const int pgv = tid < npg ? a.kv.page(b, (i64)lo + (i64)tid * DI_PAGE) : -1;
   v4i qa0 = v4i{0, 0, 0, 0}, qa1 = v4i{0, 0, 0, 0};
   if (l16 < G) {
     const int8_t* qsrc = a.q8 + q0 * 128;
     qa0 = *(const v4i*)(qsrc + l16 * 128 + grp * 16);
     qa1 = *(const v4i*)(qsrc + l16 * 128 + 64 + grp * 16);
   }
+  if (sa.add && c == 0)
+    for (int i = tid; i < G * 128; i += 256) a.out[q0 * 128 + i] = 0;
+  bool over;
+  const int S = scanned_slots(a, a.tpos, &over);
+  const int hi = ::min(lo + sa.chunk, S);
+  int32_t* cm = sa.cmax + q0 * sa.ns + c;  // head hh at cm[hh * ns]
+  report_slots(a, over, kvh == 0 && c == 0);
+  if (lo >= hi) {  // block-uniform: a chunk past the scanned slots
+    if (tid < G) cm[tid * sa.ns] = SCORE_MASKED;
+    return;
+  }
+  if (tid < npg) pg_lds[tid] = pgv;
   __syncthreads();
   int32_t* sc = a.scratch + q0 * sa.spad;
   const uint8_t* vrow = a.valid + (i64)b * a.valid_stride;
@@ -1263,17 +1275,12 @@ __global__ __launch_bounds__(256) void k_attn_split_pv(SplitArgs sa) {
   BlockRedT<4> red{red_buf, 0, 256};
   const int kvh = blockIdx.x, b = blockIdx.y, c = blockIdx.z;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, l16 = lane & 15, grp = lane >> 4;
-  bool over;
-  const int S = scanned_slots(a, a.tpos, &over);
-  const int lo = c * sa.chunk, hi = ::min(lo + sa.chunk, S);
+  const int lo = c * sa.chunk;
   const i64 q0 = (i64)b * a.n_q + kvh * G;
-  int64_t* outp = a.out + c * sa.out_stride + q0 * 128;
-  if (lo >= hi) {  // block-uniform: this chunk contributes nothing
-    for (int i = tid; i < G * 128; i += 256) outp[i] = 0;
-    return;
-  }
-  const int npg = (hi - lo + DI_PAGE - 1) / DI_PAGE;
-  if (tid < npg) pg_lds[tid] = a.kv.page(b, (i64)lo + (i64)tid * DI_PAGE);
+  int64_t* outp = a.out + (sa.add ? 0 : c * sa.out_stride) + q0 * 128;
+  // (the pages, constants and maxima load beside the device's slot count)
+  const int npg = (::min(sa.chunk, a.S - lo) + DI_PAGE - 1) / DI_PAGE;
+  const int pgv = tid < npg ? a.kv.page(b, (i64)lo + (i64)tid * DI_PAGE) : -1;
   i64 tph[G], hmax[G];
 #pragma unroll
   for (int hh = 0; hh < G; ++hh) {
@@ -1283,6 +1290,15 @@ __global__ __launch_bounds__(256) void k_attn_split_pv(SplitArgs sa) {
     for (int k = 0; k < sa.ns; ++k) m = imax(m, (i64)cmh[k]);
     hmax[hh] = m == (i64)SCORE_MASKED ? 0 : m;  // no visible slot: max := 0, every p = 0
   }
+  bool over;
+  const int S = scanned_slots(a, a.tpos, &over);
+  const int hi = ::min(lo + sa.chunk, S);
+  if (lo >= hi) {  // block-uniform: this chunk contributes nothing
+    if (!sa.add)
+      for (int i = tid; i < G * 128; i += 256) outp[i] = 0;
+    return;
+  }
+  if (tid < npg) pg_lds[tid] = pgv;
   __syncthreads();
   // V fragments of the chunk's first VPRE 64-slot steps (a step lies in one
   // page), loaded before the denominator pass
@@ -1300,16 +1316,31 @@ __global__ __launch_bounds__(256) void k_attn_split_pv(SplitArgs sa) {
 #pragma unroll
     for (int nb = 0; nb < 2; ++nb) vpre[i][nb] = vfrag(st_lo + i, nb);
   const int32_t* sc = a.scratch + q0 * sa.spad;
-  // denominators over every scanned slot of the row
+  // denominators over every scanned slot of the row: 16 bytes of scores per
+  // load and SPLIT_DL loads in flight (rows of scores start at multiples of
+  // 128 slots; a vector that reaches past S is cut there). One score per load,
+  // each waited for in turn, made this pass a chain of S / 256 round trips.
   i64 den[G];
 #pragma unroll
   for (int hh = 0; hh < G; ++hh) {
     i64 acc = 0;
     if (tph[hh] < ((i64)1 << 23)) {
       const ExpEst Ee = make_expest(tph[hh]);
-      for (int s = tid; s < S; s += 256) {
-        const int32_t x = sc[hh * sa.spad + s];
-        if (x != SCORE_MASKED) acc += dexp_est((uint32_t)(hmax[hh] - x), Ee);
+      const int32_t* row = sc + hh * sa.spad;
+      const int hm = (int)hmax[hh];
+      for (int s0 = 4 * tid; s0 < S; s0 += 1024 * SPLIT_DL) {
+        v4i x[SPLIT_DL];
+#pragma unroll
+        for (int u = 0; u < SPLIT_DL; ++u) {
+          const int s = s0 + 1024 * u;
+          x[u] = *(const v4i*)(row + (s < S ? s : s0));
+        }
+#pragma unroll
+        for (int u = 0; u < SPLIT_DL; ++u)
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            if (s0 + 1024 * u + r < S && x[u][r] != SCORE_MASKED)
+              acc += dexp_est((uint32_t)(hm - x[u][r]), Ee);
       }
     } else {
       const ExpR E = make_exp(tph[hh]);
@@ -1329,13 +1360,17 @@ __global__ __launch_bounds__(256) void k_attn_split_pv(SplitArgs sa) {
     if (tph[hh] < ((i64)1 << 23) && den[hh] < ((i64)1 << 34)) {
       const ExpEst Ee = make_expest(tph[hh]);
       const DivEst D = make_divest(den[hh], 16384.0);
-      for (int i = tid; i < n16; i += 256) {
-        i64 p = 0;
-        if (lo + i < hi) {
-          const int32_t x = sc[hh * sa.spad + lo + i];
-          if (x != SCORE_MASKED) p = rhad_est((double)dexp_est((uint32_t)(hmax[hh] - x), Ee), D);
+      for (int i = 4 * tid; i < n16; i += 1024) {  // (n16 is a multiple of 16, within the chunk)
+        const v4i x = *(const v4i*)(sc + hh * sa.spad + lo + i);
+        v4i w;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          i64 p = 0;
+          if (lo + i + r < hi && x[r] != SCORE_MASKED)
+            p = rhad_est((double)dexp_est((uint32_t)((int)hmax[hh] - x[r]), Ee), D);
+          w[r] = pack_p(p);
         }
-        ph[i] = pack_p(p);
+        *(v4i*)(ph + i) = w;
       }
     } else {
       const ExpR E = make_exp(tph[hh]);
@@ -1383,7 +1418,7 @@ __global__ __launch_bounds__(256) void k_attn_split_pv(SplitArgs sa) {
     for (int i = 0; i < 4; ++i)
       if (st0 + i < st_hi) pv_step(st0 + i, vb[i]);
   }
-  store_pv<G>(chi, clo, outp);
+  store_pv<G>(chi, clo, outp, sa.add != 0);
 }
 
 }  // namespace
@@ -1566,19 +1601,23 @@ int detllm_qkv_attn_decode_ext(const int32_t* P, int nsplit, int64_t split_strid
       valid_stride, S, s_dev, scratch, out, err, om, ext, s);
 }
 
-// Chunking of the split-S decode attention: enough chunks that the launch has
-// about 1024 blocks (four per CU; c4, 32 rows x 8 kv heads at 4096 slots:
-// 3.88 ms per step at 1024-slot chunks against 4.41 at 512, 4.20 at 2048 —
-// every block sums the whole row's denominator, so more chunks cost more),
-// chunks of at least 256 slots, a multiple of the page, within the LDS of
-// the packed p (G * chunk * 4 bytes <= 48 KiB) and SPLIT_MAX_CHUNK.
+// Chunking of the split-S decode attention: chunks of 256 to 1024 slots, cut
+// until the launch has about 256 blocks (one per CU: a CU draws no more than
+// about 32 bytes per ns, so fewer leave bandwidth unused, and every chunk
+// block sums the whole row's denominator, so more cost more); for that reason
+// also no more than 16 chunks per row, up to SPLIT_MAX_CHUNK slots each. A
+// multiple of the page, within the LDS of the packed p (G * chunk * 4 bytes
+// <= 48 KiB). us per call, 16 / 8 heads, at 256 / 512 / 1024 / 2048 slots per
+// chunk: 1 x 4000 16.1 / 17.7 / 22.3 / 32.2, 8 x 4000 29.1 / 25.9 / 25.7 /
+// 35.0, 32 x 4000 93 / 74.7 / 64.0 / 66.2, 2 x 16384 48.9 / 36.8 / 33.8 / 42.1.
 int detllm_attn_split_plan(int B, int S, int n_q, int n_kv, int* chunk, int* nsplit) {
   if (!chunk || !nsplit || B <= 0 || S <= 0 || n_q <= 0 || n_kv <= 0 || n_q % n_kv) return DI_EINVAL;
   const int G = n_q / n_kv;
   if (G > MAXG) return DI_ENOSYS;
   const i64 blocks = (i64)B * n_kv;
-  const i64 want = blocks >= 1024 ? 1 : (1024 + blocks - 1) / blocks;
-  i64 ch = ((i64)S + want - 1) / want;
+  const i64 want = blocks >= 256 ? 1 : (256 + blocks - 1) / blocks;
+  i64 ch = imin(((i64)S + want - 1) / want, 1024);
+  ch = imax(ch, ((i64)S + 15) / 16);
   ch = (ch + DI_PAGE - 1) / DI_PAGE * DI_PAGE;
   i64 cmax = DECODE_LDS_BYTES / (4 * G) / DI_PAGE * DI_PAGE;
   if (cmax > SPLIT_MAX_CHUNK) cmax = SPLIT_MAX_CHUNK;
@@ -1592,11 +1631,11 @@ int detllm_attn_split_plan(int B, int S, int n_q, int n_kv, int* chunk, int* nsp
 // detllm_qkv_epilogue with T = 1). scores: int32 [B][n_q][nsplit * chunk];
 // cmax: int32 [B][n_q][nsplit]; out: int64 partial contexts
 // [nsplit][B][n_q * 128] whose sum is detllm_attn_decode's out.
-int detllm_attn_decode_split(const int8_t* q8, const int64_t* tpos, const int8_t* kpool,
+static int attn_split_launch(const int8_t* q8, const int64_t* tpos, const int8_t* kpool,
                              const int8_t* vpool, const int32_t* table, int width,
                              const uint8_t* valid, int64_t valid_stride, int B, int S, int n_q,
                              int n_kv, const int64_t* s_dev, int chunk, int32_t* scores,
-                             int32_t* cmax, int64_t* out, int32_t* err, hipStream_t s) {
+                             int32_t* cmax, int64_t* out, bool add, int32_t* err, hipStream_t s) {
   if (B <= 0) return DI_OK;
   if (n_q <= 0 || n_kv <= 0 || n_q % n_kv || S < 1 || !kv_ok(kpool, vpool, table, width) ||
       S > (i64)width * DI_PAGE || valid_stride < S || !q8 || !tpos || !valid || !out || !scores ||
@@ -1616,6 +1655,7 @@ int detllm_attn_decode_split(const int8_t* q8, const int64_t* tpos, const int8_t
   sa.ns = ns;
   sa.spad = (i64)ns * chunk;
   sa.out_stride = (i64)B * n_q * 128;
+  sa.add = add;
   const dim3 grid(n_kv, B, ns);
 #define DI_SPLIT_LAUNCH(G_)                                                                   \
   hipLaunchKernelGGL(k_attn_split_scores<G_>, grid, dim3(256), 0, s, sa);                     \
@@ -1630,6 +1670,27 @@ int detllm_attn_decode_split(const int8_t* q8, const int64_t* tpos, const int8_t
 #undef DI_SPLIT_LAUNCH
   DI_LAUNCH_CHECK();
   return DI_OK;
+}
+
+int detllm_attn_decode_split(const int8_t* q8, const int64_t* tpos, const int8_t* kpool,
+                             const int8_t* vpool, const int32_t* table, int width,
+                             const uint8_t* valid, int64_t valid_stride, int B, int S, int n_q,
+                             int n_kv, const int64_t* s_dev, int chunk, int32_t* scores,
+                             int32_t* cmax, int64_t* out, int32_t* err, hipStream_t s) {
+  return attn_split_launch(q8, tpos, kpool, vpool, table, width, valid, valid_stride, B, S, n_q,
+                           n_kv, s_dev, chunk, scores, cmax, out, false, err, s);
+}
+
+// detllm_attn_decode_split with the partials added up: out [B][n_q * 128] as
+// detllm_attn_decode writes it.
+int detllm_attn_decode_split_sum(const int8_t* q8, const int64_t* tpos, const int8_t* kpool,
+                                 const int8_t* vpool, const int32_t* table, int width,
+                                 const uint8_t* valid, int64_t valid_stride, int B, int S,
+                                 int n_q, int n_kv, const int64_t* s_dev, int chunk,
+                                 int32_t* scores, int32_t* cmax, int64_t* out, int32_t* err,
+                                 hipStream_t s) {
+  return attn_split_launch(q8, tpos, kpool, vpool, table, width, valid, valid_stride, B, S, n_q,
+                           n_kv, s_dev, chunk, scores, cmax, out, true, err, s);
 }
 
 }  // extern "C"

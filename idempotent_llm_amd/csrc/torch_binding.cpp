@@ -126,7 +126,7 @@ const Entry ENTRIES[] = {
     DI_ENTRY(detllm_igemv_plan), DI_ENTRY(detllm_attn_split_plan), DI_ENTRY(detllm_transpose_i8), DI_ENTRY(detllm_pack_nt),
     DI_ENTRY(detllm_greedy_pick), DI_ENTRY(detllm_greedy_pick_noalloc),
     DI_ENTRY(detllm_logits_digest), DI_ENTRY(detllm_embed_normq), DI_ENTRY(detllm_residual_normq),
-    DI_ENTRY(detllm_norm_quant), DI_ENTRY(detllm_attn_decode_split),
+    DI_ENTRY(detllm_norm_quant), DI_ENTRY(detllm_attn_decode_split), DI_ENTRY(detllm_attn_decode_split_sum),
     DI_ENTRY(detllm_igemv_resnormq), DI_ENTRY(detllm_igemv_merge),
     DI_ENTRY(detllm_igemv_merge_ext), DI_ENTRY(detllm_swiglu_quant),
     DI_ENTRY(detllm_igemv_swiglu), DI_ENTRY(detllm_merge_rowcol), DI_ENTRY(detllm_merge_ext),
@@ -387,11 +387,28 @@ Tensor op_attn_decode(const Tensor& q8, const Tensor& tpos, const Tensor& kpool,
                       const Tensor& vpool, const Tensor& table, const Tensor& valid, int64_t S,
                       const Tensor& err) {
   const int64_t B = q8.size(0), n_q = q8.size(1), n_kv = kpool.size(1), G = n_q / n_kv;
+  Tensor out = empty({B, n_q * 128}, at::kLong, q8);
+  const Tensor qc = q8.contiguous(), tc = tpos.contiguous(), v = valid.view(at::kByte);
+  // Long rows of few (row, kv head) pairs: a block per pair leaves most CUs
+  // idle, so the rows are cut into chunks. us per call, one block / chunks:
+  // 1 x 1024 slots 17.6 / 13.6, 8 x 1024 19.4 / 15.3, 8 x 4096 58.2 / 26; at
+  // 576 slots, and from 32 rows on, the two are even.
+  if (B > 0 && S >= 768 && B * n_kv <= 128) {
+    int chunk = 0, ns = 0;
+    check(detllm_attn_split_plan((int)B, (int)S, (int)n_q, (int)n_kv, &chunk, &ns),
+          "detllm_attn_split_plan");
+    const Tensor scores = empty({B, n_q, (int64_t)ns * chunk}, at::kInt, q8);
+    const Tensor cmax = empty({B, n_q, ns}, at::kInt, q8);
+    DI_RUN(detllm_attn_decode_split_sum, ptr<int8_t>(qc), i64(tc), ptr<int8_t>(kpool),
+           ptr<int8_t>(vpool), ptr<int32_t>(table), (int)table.size(1), ptr<uint8_t>(v),
+           valid.size(1), (int)B, (int)S, (int)n_q, (int)n_kv, nullptr, chunk,
+           ptr<int32_t>(scores), ptr<int32_t>(cmax), ptr<int64_t>(out), ptr<int32_t>(err));
+    mutated(err);
+    return out;
+  }
   const int64_t Spad = (S + 15) / 16 * 16;
   OptTensor scratch;
   if (G * Spad * 4 > 48 * 1024) scratch = empty({B, n_q, Spad}, at::kInt, q8);
-  Tensor out = empty({B, n_q * 128}, at::kLong, q8);
-  const Tensor qc = q8.contiguous(), tc = tpos.contiguous(), v = valid.view(at::kByte);
   DI_RUN(detllm_attn_decode, ptr<int8_t>(qc), i64(tc), ptr<int8_t>(kpool), ptr<int8_t>(vpool),
          ptr<int32_t>(table), (int)table.size(1), ptr<uint8_t>(v), valid.size(1), (int)B, (int)S,
          (int)n_q, (int)n_kv, nullptr, ptr<int32_t>(scratch), ptr<int64_t>(out), ptr<int32_t>(err));

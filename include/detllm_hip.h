@@ -358,8 +358,19 @@ int detllm_attn_decode_split(const int8_t* q8, const int64_t* tpos, const int8_t
                              int n_kv, const int64_t* s_dev, int chunk, int32_t* scores,
                              int32_t* cmax, int64_t* out, int32_t* err, hipStream_t s);
 
+/* detllm_attn_decode_split with the chunks' partials added up on the device
+ * (the scores launch zeroes out, the second adds to it): out [B][n_q * 128] as
+ * detllm_attn_decode writes it, the same integers. */
+int detllm_attn_decode_split_sum(const int8_t* q8, const int64_t* tpos, const int8_t* kpool,
+                                 const int8_t* vpool, const int32_t* table, int width,
+                                 const uint8_t* valid, int64_t valid_stride, int B, int S,
+                                 int n_q, int n_kv, const int64_t* s_dev, int chunk,
+                                 int32_t* scores, int32_t* cmax, int64_t* out, int32_t* err,
+                                 hipStream_t s);
+
 /* The chunking detllm_attn_decode_split is tuned for at (B, S, n_q, n_kv):
- * about 1024 blocks, chunks of 256 slots or more. Writes *chunk, *nsplit. */
+ * about 256 blocks, chunks of 256 to 1024 slots (more for rows past 16384, at
+ * most 16 chunks up to 4096 slots each). Writes *chunk, *nsplit. */
 int detllm_attn_split_plan(int B, int S, int n_q, int n_kv, int* chunk, int* nsplit);
 
 /* Per-step bookkeeping of the graph-captured decode (src/detllm/graphed.py:

@@ -681,3 +681,57 @@ def test_prefill_attention_resident_pages(T, S_past):
          vmask.view(torch.uint8), width * 128, B, T, S_past, n_q, n_kv, out)
     bad = np.argwhere(out.cpu().numpy() != want)
     assert bad.size == 0, f"{len(bad)} mismatches, first at {bad[0].tolist()}"
+
+
+@pytest.mark.parametrize("name", list(SPLIT_CASES))
+def test_split_decode_summed(name):
+    """detllm_attn_decode_split_sum (the partials added on the device) against
+    the oracle, twice into the same buffer (the launch zeroes it itself)."""
+    from idempotent_llm_amd._lib import call
+    B, n_q, n_kv, S, cap, seed, lo, hi, extra = SPLIT_CASES[name]
+    print(f"[split decode summed {name}: B={B} n_q={n_q} n_kv={n_kv} S={S}]", flush=True)
+    q8, kc, vc, valid, sm, sk, tpos = _prefill_case(B, n_q, n_kv, 1, S - 1, cap, seed, lo, hi,
+                                                    **extra)
+    want = _prefill_oracle(q8, kc, vc, valid, sm, sk, S - 1)[:, 0]
+    d = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()
+    kp, vp, table, width, vmask = paged(kc, vc, valid, seed=seed)
+    ns = -(-S // 256)
+    out = torch.full((B, n_q * 128), -7, dtype=I64, device="cuda")
+    for _ in range(2):
+        scores = torch.full((B, n_q, ns * 256), 0x7F7F7F7F, dtype=torch.int32, device="cuda")
+        cmax = torch.full((B, n_q, ns), 0x7F7F7F7F, dtype=torch.int32, device="cuda")
+        call("detllm_attn_decode_split_sum", d(q8[:, :, 0]), d(tpos[:, :, 0, 0]), kp, vp, table,
+             width, vmask.view(torch.uint8), width * 128, B, S, n_q, n_kv, None, 256, scores,
+             cmax, out, None)
+        assert np.array_equal(out.cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("S", [1, 767, 768, 769, 1023, 1025, 2049, 4099])
+@pytest.mark.parametrize("B,n_q,n_kv", [(1, 16, 8), (17, 16, 8), (2, 8, 1)])
+def test_attn_decode_op_routes(S, B, n_q, n_kv):
+    """The registered decode attention on both sides of its chunking rule
+    (slots, rows x kv heads) gives the one-block kernel's context, with a
+    ragged mask, a dead row and slot counts that end inside a vector of
+    scores; a row of page-table width beyond the scanned slots stays unread."""
+    from idempotent_llm_amd import torch_ops  # noqa: F401
+    from idempotent_llm_amd._lib import call
+    print(f"[attn_decode op S={S} B={B} n_q={n_q} n_kv={n_kv}]", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(S + B)
+    w = -(-S // 128) + 1
+    i8 = lambda *s: torch.randint(-128, 128, s, dtype=torch.int8, device="cuda", generator=g)
+    kp, vp = i8(B * w, n_kv, 128, 128), i8(B * w, n_kv, 128, 128)
+    table = torch.randperm(B * w, device="cuda", generator=g).to(torch.int32).view(B, w)
+    table[:, -1] = -1
+    valid = torch.rand(B, w * 128, device="cuda", generator=g) < 0.8
+    if B > 1:
+        valid[1, :S] = False
+    q8 = i8(B, n_q, 128)
+    tpos = torch.randint(1, 1 << 16, (B, n_q), device="cuda", generator=g)
+    tpos[0, 0] = 1 << 40
+    err = torch.zeros(1, dtype=torch.int32, device="cuda")
+    got = torch.ops.detllm_rocm.attn_decode(q8, tpos, kp, vp, table, valid, S, err)
+    want = torch.full((B, n_q * 128), -7, dtype=I64, device="cuda")
+    scratch = torch.empty(B, n_q, (S + 15) // 16 * 16, dtype=torch.int32, device="cuda")
+    call("detllm_attn_decode", q8, tpos, kp, vp, table, w, valid.view(torch.uint8), w * 128, B, S,
+         n_q, n_kv, None, scratch, want, err)
+    assert torch.equal(got, want) and int(err) == 0
