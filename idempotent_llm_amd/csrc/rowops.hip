@@ -572,8 +572,10 @@ struct ResNormArgs {
 };
 
 // MODE: the row's mode when the launch fixes it (the kernel then holds that
-// path only: less code to fetch per launch), else -1 (a.mode decides).
-template <int VPT, class Red, int MODE = -1>
+// path only: less code to fetch per launch), else -1 (a.mode decides). KF: the
+// partials of the product loaded with the row's first loads (load_rows_i32_first;
+// loads past nsplit repeat the last one, so a launch of one partial takes 1).
+template <int VPT, class Red, int MODE = -1, int KF = 4>
 __device__ __forceinline__ void residual_normq_row(const ResNormArgs& a, int r, Red& red) {
   const int mode = MODE >= 0 ? MODE : a.mode;
   const int C = a.C;
@@ -595,7 +597,6 @@ __device__ __forceinline__ void residual_normq_row(const ResNormArgs& a, int r, 
     }
     i64 row_k = a.row_k[r], row_m = a.row_m[r];
     const i64 k_res = (a.k_res_in ? a.k_res_in : a.k_res)[r];
-    constexpr int KF = 4;
     int32_t t[KF][1][VPT];
     const i64 offs[1] = {off};
     load_rows_i32_first<KF, 1, VPT>(t, a.P, a.nsplit, a.split_stride, offs, C, red);
@@ -686,7 +687,7 @@ __global__ __launch_bounds__(NT) void k_residual_normq(ResNormArgs a) {
 }
 
 // The GEMM residual add (mode 1) only.
-template <int VPT, int NT = RT_WIDE, bool WARM = false>
+template <int VPT, int NT = RT_WIDE, bool WARM = false, int KF = 4>
 __global__ __launch_bounds__(NT) void k_residual_add_normq(ResNormArgs a) {
   keep_hidden_args();
   __shared__ i64 red_buf[32];
@@ -695,20 +696,21 @@ __global__ __launch_bounds__(NT) void k_residual_add_normq(ResNormArgs a) {
     return;
   }
   RowRed<NT> red{red_buf, 0, a.nt};
-  residual_normq_row<VPT, decltype(red), 1>(a, (int)blockIdx.x - (WARM ? L2WARM_BLOCKS : 0), red);
+  residual_normq_row<VPT, decltype(red), 1, KF>(a, (int)blockIdx.x - (WARM ? L2WARM_BLOCKS : 0),
+                                                 red);
 }
 
 // Many rows (prefill): one wave per row, four rows per block, every
 // reduction a DPP reduction within the wave (no LDS round trip, no barrier),
 // so more rows are in flight per CU than with a block per row.
-template <int VPT, int MODE>
+template <int VPT, int MODE, int KF = 4>
 __global__ __launch_bounds__(256) void k_residual_normq_w(ResNormArgs a, int R) {
   keep_hidden_args();
   // (wave-uniform: the row's buffer views live in scalar registers)
   const int r = __builtin_amdgcn_readfirstlane((int)blockIdx.x * 4 + (int)(threadIdx.x >> 6));
   if (r >= R) return;  // whole waves
   WaveRed red;
-  residual_normq_row<VPT, WaveRed, MODE>(a, r, red);
+  residual_normq_row<VPT, WaveRed, MODE, KF>(a, r, red);
 }
 
 struct SwigluArgs {
@@ -1890,15 +1892,23 @@ void launch_pro(const ProGemv& g, int ni, int ksplit, const ResNormArgs& ra, con
 // lane is long; up to 640 rows a block per row (four columns per lane) fits
 // the chip two or three blocks per CU and is done sooner: residual rows 320 /
 // 512 / 700 / 1024 / 2048 take 7.3 / 7.6 / 8.8 / 10.1 / 14.4 us as blocks, 8.6
-// / 8.8 / 9.1 / 9.3 / 12.5 as waves.
+// / 8.8 / 9.1 / 9.3 / 12.5 as waves. (The norm-quant alone, a shorter chain,
+// takes the wave at every size: 512 rows 6.0 us.)
 constexpr int ROWS_WAVE_MIN = 641;
 template <int MODE>
 static bool rows_wave_launch(int R, int C, hipStream_t s, ResNormArgs& a) {
-  if (R < ROWS_WAVE_MIN || (C != 512 && C != 1024)) return false;
+  if (R <= (MODE == 1 ? ROWS_WAVE_MIN - 1 : 64) || (C != 512 && C != 1024)) return false;
   a.nt = 64;
   const dim3 grid((unsigned)((R + 3) / 4));
-  if (C == 1024) hipLaunchKernelGGL((k_residual_normq_w<16, MODE>), grid, dim3(256), 0, s, a, R);
-  else hipLaunchKernelGGL((k_residual_normq_w<8, MODE>), grid, dim3(256), 0, s, a, R);
+  // (one partial: its loads alone; 2048 rows 12.4 -> 11.6 us, 4096 20.7 -> 19.4)
+  const bool one = MODE != 1 || a.nsplit == 1;
+  if (C == 1024) {
+    if (one) hipLaunchKernelGGL((k_residual_normq_w<16, MODE, 1>), grid, dim3(256), 0, s, a, R);
+    else hipLaunchKernelGGL((k_residual_normq_w<16, MODE, 4>), grid, dim3(256), 0, s, a, R);
+  } else {
+    if (one) hipLaunchKernelGGL((k_residual_normq_w<8, MODE, 1>), grid, dim3(256), 0, s, a, R);
+    else hipLaunchKernelGGL((k_residual_normq_w<8, MODE, 4>), grid, dim3(256), 0, s, a, R);
+  }
   return true;
 }
 
@@ -1945,7 +1955,13 @@ int detllm_residual_normq(const int32_t* P, int nsplit, int64_t split_stride, in
   a.col_m = col_m; a.col_k = col_k; a.tb = tb;
   a.h = h; a.k_res = k_res; a.sm_m = sm_m; a.sm_k = sm_k; a.x8 = x8; a.xm = xm; a.xk = xk;
   a.warm = warm_for(R, next_w, next_n, next_k, next_ksplit);
-  if (!rows_wave_launch<1>(R, C, s, a)) DI_WARM_OR_ROWS(R, C, k_residual_add_normq, s, a);
+  if (rows_wave_launch<1>(R, C, s, a)) {
+  } else if (R > 64 && C <= 1024 && nsplit == 1) {
+    a.nt = 256;
+    hipLaunchKernelGGL((k_residual_add_normq<4, 256, false, 1>), dim3(R), dim3(256), 0, s, a);
+  } else {
+    DI_WARM_OR_ROWS(R, C, k_residual_add_normq, s, a);
+  }
   DI_LAUNCH_CHECK();
   return DI_OK;
 }
