@@ -446,6 +446,7 @@ __global__ __launch_bounds__(256, 2) void k_attn_prefill(PrefillArgs a) {
     for (int c = 0; c < 2; ++c) ocs[c] = mfma16(ones, vc[c], ocs[c]);
   }); });
   // column sums: every row of ocs[c] holds sum_s v[s][32 wave + 16 c + qi]
+  if (resident) __syncthreads();  // every wave has read its nfull there (no barrier since)
   if (g == 0) {
     csum_lds[32 * wave + qi] = ocs[0][0];
     csum_lds[32 * wave + 16 + qi] = ocs[1][0];
