@@ -886,7 +886,10 @@ int detllm_igemm_nt(const int8_t* A, const int8_t* B, int32_t* C, int M, int N, 
   if (M <= 0 || N <= 0 || batch <= 0) return DI_OK;
   if (K <= 0 || (K % 16) != 0 || K > 131071 || !A || !B || !C) return DI_EINVAL;
   if (batch > 65535) return DI_ERANGE;
-  if (K % G2_BK == 0) {  // (M <= 64: batched products, one matrix of few rows takes the skinny kernels)
+  // M <= 64: batched products (one matrix of few rows takes the skinny
+  // kernels); their direct-to-LDS loads need 16-byte operands, k_gemm_nt's do not
+  const bool aligned = (((uintptr_t)A | (uintptr_t)B | (uintptr_t)sA | (uintptr_t)sB) & 15) == 0;
+  if (K % G2_BK == 0 && (M > 64 || aligned)) {
     // Tile shape by tile count, from sweeps of every shape over the model's
     // four products at 65 to 2048 rows. n = tiles of 128 x 64; us of the taken
     // shape against 128 x 64 (one block per CU):

@@ -244,9 +244,10 @@ Tensor op_int_gemm(const Tensor& a, const Tensor& b) {
   shape.back() = N;
   if (M == 0 || N == 0) return at::zeros(shape, a.options().dtype(at::kInt));
   // few rows of one matrix take the skinny kernels (K in steps of 16), the
-  // rest the tiled one, at its best in whole 128-byte slices of K
+  // rest the tiled one, at its best in whole 128-byte slices of K (unless
+  // those pass the largest K of an int32 sum, 131071)
   const bool skinny = a.dim() == 2 && M <= 64;
-  const int64_t step = skinny ? 16 : 128;
+  const int64_t step = skinny || (K + 127) / 128 * 128 > 131071 ? 16 : 128;
   const int64_t Kp = std::max(step, (K + step - 1) / step * step);
   int64_t batch = 1;
   for (int64_t i = 0; i < a.dim() - 2; ++i) batch *= a.size(i);

@@ -103,3 +103,25 @@ def test_int_gemm_batched(lead, M, K, N):
     b = torch.randint(-128, 128, (*lead, K, N), dtype=torch.int8, device="cuda")
     want = torch.matmul(a.cpu().double(), b.cpu().double()).to(torch.int32)
     assert torch.equal(int_gemm(a, b, "rocm").cpu(), want)
+
+
+@pytest.mark.parametrize("K", [130943, 130945, 131056])
+def test_int_gemm_longest_k(K):
+    """Whole 128-byte slices of these K pass the largest sum (131071) from
+    130945 on, where K is padded to 16 only."""
+    from idempotent_llm_amd.backends import int_gemm
+    print(f"[int_gemm longest K={K}]", flush=True)
+    a, b = _i8(1, 65, K), _i8(2, K, 40)
+    assert torch.equal(int_gemm(a, b, "rocm"), (a.double() @ b.double()).to(torch.int32))
+
+
+def test_few_rows_at_any_alignment():
+    """detllm_igemm_nt of few rows takes operands at any address."""
+    from idempotent_llm_amd._lib import call
+    M, N, K = 40, 70, 256
+    print("[igemm few rows, operands off by 4 bytes]", flush=True)
+    a = _i8(3, M * K + 16)[4:4 + M * K].view(M, K)
+    w = _i8(4, N * K + 16)[4:4 + N * K].view(N, K)
+    out = torch.empty(M, N, dtype=torch.int32, device="cuda")
+    call("detllm_igemm_nt", a, w, out, M, N, K, 1, 0, 0, 0)
+    assert torch.equal(out, _want(a, w))
