@@ -229,6 +229,10 @@ Tensor empty(at::IntArrayRef shape, at::ScalarType dt, const Tensor& like) {
 void mutated(const Tensor& t) {
   if (!t.is_inference()) t.unsafeGetTensorImpl()->bump_version();
 }
+// Operands of another rank are refused, as unpacking their shape did.
+void rank(const Tensor& t, int64_t n, const char* op) {
+  TORCH_CHECK_VALUE(t.dim() == n, op, ": expected ", n, " dimensions, got ", t.dim());
+}
 T3 rows_out(int64_t R, int64_t C, const Tensor& like) {
   return {empty({R, C}, at::kChar, like), empty({R}, at::kLong, like), empty({R}, at::kLong, like)};
 }
@@ -278,6 +282,7 @@ Tensor op_isqrt(const Tensor& a) { return scalar_op(0, a); }
 Tensor op_ilog2(const Tensor& a) { return scalar_op(1, a); }
 
 Tensor op_greedy_pick(const Tensor& logits, const Tensor& head_m) {
+  rank(logits, 2, "greedy_pick");
   constexpr int64_t chunk = 2048;
   const int64_t R = logits.size(0), V = logits.size(1), nch = (V + chunk - 1) / chunk;
   Tensor pv = empty({R, nch}, at::kLong, logits), pi = empty({R, nch}, at::kLong, logits);
@@ -303,6 +308,7 @@ std::tuple<Tensor, Tensor, Tensor, Tensor, Tensor> op_embed_normq(
 }
 
 T3 op_norm_quant(const Tensor& h, const OptTensor& sm_m, int64_t sm_k) {
+  rank(h, 2, "norm_quant");
   const int64_t R = h.size(0), C = h.size(1);
   auto [x8, xm, xk] = rows_out(R, C, h);
   const Tensor hc = h.contiguous();
@@ -314,6 +320,7 @@ T3 op_norm_quant(const Tensor& h, const OptTensor& sm_m, int64_t sm_k) {
 T3 op_residual_normq(const Tensor& P, const Tensor& row_m, const Tensor& row_k,
                      const Tensor& col_m, int64_t col_k, int64_t tb, const Tensor& h,
                      const Tensor& k_res, const OptTensor& sm_m, int64_t sm_k) {
+  rank(P, 3, "residual_normq");
   const int64_t ns = P.size(0), R = P.size(1), C = P.size(2);
   auto [x8, xm, xk] = rows_out(R, C, P);
   const Tensor Pc = P.contiguous();
@@ -328,6 +335,7 @@ T3 op_residual_normq(const Tensor& P, const Tensor& row_m, const Tensor& row_k,
 T3 op_swiglu_quant(const Tensor& P, const Tensor& xm, const Tensor& xk, const Tensor& gate_m,
                    int64_t gate_k, const Tensor& up_m, int64_t up_k, const Tensor& ds_m,
                    int64_t ds_k) {
+  rank(P, 3, "swiglu_quant");
   const int64_t ns = P.size(0), R = P.size(1), C2 = P.size(2), I = C2 / 2;
   auto [y8, ym, yk] = rows_out(R, I, P);
   const Tensor Pc = P.contiguous();
@@ -339,6 +347,7 @@ T3 op_swiglu_quant(const Tensor& P, const Tensor& xm, const Tensor& xk, const Te
 
 T3 op_merge_rowcol(const Tensor& attn, const Tensor& os_m, int64_t os_k, const Tensor& col_m,
                    int64_t col_k) {
+  rank(attn, 2, "merge_rowcol");
   const int64_t R = attn.size(0), C = attn.size(1);
   auto [a8, am, ak] = rows_out(R, C, attn);
   const Tensor ac = attn.contiguous();
@@ -356,6 +365,7 @@ T2 op_qkv_epilogue(const Tensor& P, int64_t B, int64_t T, int64_t n_q, int64_t n
                    const Tensor& vq_k, const Tensor& cos_t, const Tensor& sin_t,
                    const Tensor& kpool, const Tensor& vpool, const Tensor& table,
                    int64_t slot_base, const Tensor& err) {
+  rank(P, 3, "qkv_epilogue");
   const int64_t ns = P.size(0), R = P.size(1);
   Tensor q8 = empty({B, n_q, T, 128}, at::kChar, P), tpos = empty({B, n_q, T}, at::kLong, P);
   const Tensor Pc = P.contiguous(), pos = positions.contiguous();
@@ -375,6 +385,7 @@ T2 op_qkv_epilogue(const Tensor& P, int64_t B, int64_t T, int64_t n_q, int64_t n
 Tensor op_attn_prefill(const Tensor& q8, const Tensor& tpos, const Tensor& kpool,
                        const Tensor& vpool, const Tensor& table, const Tensor& valid,
                        int64_t S_past) {
+  rank(q8, 4, "attn_prefill");
   const int64_t B = q8.size(0), n_q = q8.size(1), T = q8.size(2), n_kv = kpool.size(1);
   Tensor out = empty({B, T, n_q * 128}, at::kLong, q8);
   const Tensor qc = q8.contiguous(), tc = tpos.contiguous(), v = valid.view(at::kByte);
@@ -387,7 +398,9 @@ Tensor op_attn_prefill(const Tensor& q8, const Tensor& tpos, const Tensor& kpool
 Tensor op_attn_decode(const Tensor& q8, const Tensor& tpos, const Tensor& kpool,
                       const Tensor& vpool, const Tensor& table, const Tensor& valid, int64_t S,
                       const Tensor& err) {
-  const int64_t B = q8.size(0), n_q = q8.size(1), n_kv = kpool.size(1), G = n_q / n_kv;
+  const int64_t B = q8.size(0), n_q = q8.size(1), n_kv = kpool.size(1);
+  TORCH_CHECK_VALUE(n_kv > 0, "attn_decode: no kv heads");
+  const int64_t G = n_q / n_kv;
   Tensor out = empty({B, n_q * 128}, at::kLong, q8);
   const Tensor qc = q8.contiguous(), tc = tpos.contiguous(), v = valid.view(at::kByte);
   // Long rows of few (row, kv head) pairs: a block per pair leaves most CUs

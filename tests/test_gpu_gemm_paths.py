@@ -125,3 +125,21 @@ def test_few_rows_at_any_alignment():
     out = torch.empty(M, N, dtype=torch.int32, device="cuda")
     call("detllm_igemm_nt", a, w, out, M, N, K, 1, 0, 0, 0)
     assert torch.equal(out, _want(a, w))
+
+
+def test_operators_refuse_other_ranks():
+    """Operands of another rank raise before any launch."""
+    from idempotent_llm_amd import torch_ops  # noqa: F401
+    ops = torch.ops.detllm_rocm
+    i32, i64, i8 = (torch.zeros(2, 2, 2, 2, 128, dtype=t, device="cuda")
+                    for t in (torch.int32, torch.int64, torch.int8))
+    v = i64.view(-1)
+    for f in (lambda: ops.greedy_pick(i32[0], v), lambda: ops.norm_quant(i32[0], None, 0),
+              lambda: ops.swiglu_quant(i32[0], v, v, v, 0, v, 0, v, 0),
+              lambda: ops.merge_rowcol(i64[0], v, 0, v, 0),
+              lambda: ops.residual_normq(i32[0], v, v, v, 0, 20, i32[0, 0, 0], v, None, 0),
+              lambda: ops.attn_prefill(i8, v, i8, i8, i32, i8[0, 0, 0].bool(), 0)):
+        with pytest.raises(ValueError):
+            f()
+    with pytest.raises(ValueError):
+        ops.attn_decode(i8[0, 0], v, i8[:, :0], i8, i32[0, 0, 0], i8[0, 0, 0].bool(), 1, i32)
