@@ -237,7 +237,23 @@ T3 rows_out(int64_t R, int64_t C, const Tensor& like) {
   return {empty({R, C}, at::kChar, like), empty({R}, at::kLong, like), empty({R}, at::kLong, like)};
 }
 
+// What the packing and product kernels index by a's shape alone: one-byte
+// elements, one K, b's matrices one for all or one each, one device.
+void check_int_gemm(const Tensor& a, const Tensor& b) {
+  TORCH_CHECK_VALUE(a.element_size() == 1 && b.element_size() == 1,
+                    "int_gemm: expected int8 operands, got ", a.scalar_type(), " and ",
+                    b.scalar_type());
+  TORCH_CHECK_VALUE(a.dim() >= 2 && b.dim() >= 2 && a.size(-1) == b.size(-2) &&
+                        (b.dim() == 2 || a.sizes().slice(0, a.dim() - 2) ==
+                                             b.sizes().slice(0, b.dim() - 2)),
+                    "int_gemm: expected [*, M, K] and [K, N] or [*, K, N], got ", a.sizes(),
+                    " and ", b.sizes());
+  TORCH_CHECK_VALUE(a.device() == b.device(), "int_gemm: operands on ", a.device(), " and ",
+                    b.device());
+}
+
 Tensor op_int_gemm(const Tensor& a, const Tensor& b) {
+  check_int_gemm(a, b);
   if (b.dim() == 2 && a.dim() > 2) {
     auto lead = a.sizes().vec();
     lead.back() = b.size(-1);

@@ -57,7 +57,14 @@ def _op(schema):
 @_op("int_gemm(Tensor a, Tensor b) -> Tensor")
 def int_gemm(a, b):
     """backends.int_gemm(a, b, "rocm"): a [*, M, K] int8 x b [*, K, N] int8 ->
-    int32 [*, M, N] (a 2-D b is shared by every leading index)."""
+    int32 [*, M, N] (a 2-D b is shared by every leading index). Other shapes
+    raise ValueError, traced or run."""
+    torch._check_value(a.dim() >= 2 and b.dim() >= 2, lambda: "int_gemm: operands of rank 2 or more")
+    torch._check_value(b.dim() == 2 or a.dim() == b.dim(), lambda: "int_gemm: leading dimensions differ")
+    torch._check_value(a.shape[-1] == b.shape[-2], lambda: "int_gemm: K differs")
+    if b.dim() > 2:
+        for m, n in zip(a.shape[:-2], b.shape[:-2]):
+            torch._check_value(m == n, lambda: "int_gemm: leading dimensions differ")
     return a.new_empty(tuple(a.shape[:-1]) + (b.shape[-1],), dtype=torch.int32)
 
 

@@ -47,3 +47,42 @@ def test_operators_mutate_what_they_declare():
         assert torch.Tag.pt2_compliant_tag in op.tags
         assert torch._C._dispatch_has_kernel_for_dispatch_key(f"detllm_rocm::{name}", "CUDA")
         assert not torch._C._dispatch_has_kernel_for_dispatch_key(f"detllm_rocm::{name}", "CPU")
+
+
+# shapes int_gemm must refuse: a b of fewer or more rows than a's K (within
+# and beyond the padded K), a batched b against one matrix, other batches
+BAD_INT_GEMM = [((3, 16), (8, 5)), ((3, 16), (17, 5)), ((3, 100), (129, 5)), ((65, 200), (1, 40)),
+                ((0, 16), (8, 5)), ((3, 16), (2, 16, 5)), ((4, 3, 16), (2, 16, 5)),
+                ((2, 3, 3, 16), (3, 2, 16, 5)), ((4, 3, 16), (8, 5)), ((2, 3, 16), (2, 8, 5)),
+                ((16,), (16, 5)), ((3, 16), (16,))]
+
+
+@pytest.mark.parametrize("sa,sb", BAD_INT_GEMM)
+def test_int_gemm_refuses_other_shapes(sa, sb):
+    """The operator's kernels index b by a's shape, so operands that do not
+    fit raise before any allocation or launch: called as the operator itself
+    (the native kernel, on host tensors: no GPU work is reached) and traced."""
+    import torch
+    from torch._subclasses.fake_tensor import FakeTensorMode
+
+    from idempotent_llm_amd import torch_ops  # noqa: F401
+    op = torch.ops.detllm_rocm.int_gemm.default
+    key = torch._C.DispatchKeySet(torch._C.DispatchKey.CUDA)
+    a, b = torch.zeros(sa, dtype=torch.int8), torch.zeros(sb, dtype=torch.int8)
+    with pytest.raises(ValueError):
+        op.redispatch(key, a, b)
+    with FakeTensorMode(), pytest.raises(ValueError):
+        op(torch.empty(sa, dtype=torch.int8, device="cuda"),
+           torch.empty(sb, dtype=torch.int8, device="cuda"))
+
+
+def test_int_gemm_refuses_wide_elements():
+    import torch
+
+    from idempotent_llm_amd import torch_ops  # noqa: F401
+    op = torch.ops.detllm_rocm.int_gemm.default
+    key = torch._C.DispatchKeySet(torch._C.DispatchKey.CUDA)
+    i8, i32 = torch.zeros(16, 16, dtype=torch.int8), torch.zeros(16, 16, dtype=torch.int32)
+    for a, b in ((i8, i32), (i32, i8)):
+        with pytest.raises(ValueError):
+            op.redispatch(key, a, b)
