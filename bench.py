@@ -279,12 +279,14 @@ def gemv_rooflines(model, B: int):
 
 def split_attention_case(model, B: int = 32, S: int = 4096, seed: int = 4):
     """The split-S decode attention at config c4's decode shape (B rows
-    scanning S slots, the model's head counts) on a random paged cache with
-    every slot valid. Returns (launch fn, algorithmic bytes per call, plan):
-    the bytes are the K and V bytes scanned, the queries, DI-Exp constants and
-    the int64 partial contexts written."""
+    scanning S slots, the model's head counts) in chunks of 1024 slots, on a
+    random paged cache with every slot valid. (The model itself takes the
+    one-block kernel for this many rows: detllm_attn_split_plan.) Returns
+    (launch fn, algorithmic bytes per call, (chunk, nsplit)): the bytes are
+    the K and V bytes scanned, the queries, DI-Exp constants and the int64
+    partial contexts written."""
     import torch
-    from idempotent_llm_amd._lib import attn_split_plan, call
+    from idempotent_llm_amd._lib import call
     from idempotent_llm_amd.kvcache import pages_from_contiguous
     nq, nkv, hd = model.n_q, model.n_kv, model.hd
     g = torch.Generator(device="cuda").manual_seed(seed)
@@ -295,7 +297,7 @@ def split_attention_case(model, B: int = 32, S: int = 4096, seed: int = 4):
     valid = torch.ones(B, S, dtype=torch.uint8, device="cuda")
     q8 = torch.randint(-128, 128, (B, nq, hd), device="cuda", dtype=torch.int8, generator=g)
     tpos = torch.randint(1, 1 << 22, (B, nq), device="cuda", dtype=torch.int64, generator=g)
-    chunk, ns = attn_split_plan(B, S, nq, nkv)
+    chunk, ns = 1024, -(-S // 1024)
     scores = torch.empty(B, nq, ns * chunk, dtype=torch.int32, device="cuda")
     cmax = torch.empty(B, nq, ns, dtype=torch.int32, device="cuda")
     out = torch.empty(ns, B, nq * hd, dtype=torch.int64, device="cuda")
@@ -324,7 +326,7 @@ def split_attention_roofline(model):
             "chunk": chunk, "nsplit": ns, "bytes_per_call": int(nbytes),
             "avg_call_us": round(us, 3),
             "timing": "HIP events around 20 replays of a graph of one split-S attention call "
-                      "(one layer of c4's decode at 4096 slots)"}
+                      "(32 rows x 4096 slots in 1024-slot chunks)"}
 
 
 def kernel_probe(model, B: int, reps: int = 3):

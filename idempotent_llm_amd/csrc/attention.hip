@@ -1602,26 +1602,45 @@ int detllm_qkv_attn_decode_ext(const int32_t* P, int nsplit, int64_t split_strid
       valid_stride, S, s_dev, scratch, out, err, om, ext, s);
 }
 
-// Chunking of the split-S decode attention: chunks of 256 to 1024 slots, cut
-// until the launch has about 256 blocks (one per CU: a CU draws no more than
-// about 32 bytes per ns, so fewer leave bandwidth unused, and every chunk
-// block sums the whole row's denominator, so more cost more); for that reason
-// also no more than 16 chunks per row, up to SPLIT_MAX_CHUNK slots each. A
-// multiple of the page, within the LDS of the packed p (G * chunk * 4 bytes
-// <= 48 KiB). us per call, 16 / 8 heads, at 256 / 512 / 1024 / 2048 slots per
-// chunk: 1 x 4000 16.1 / 17.7 / 22.3 / 32.2, 8 x 4000 29.1 / 25.9 / 25.7 /
-// 35.0, 32 x 4000 93 / 74.7 / 64.0 / 66.2, 2 x 16384 48.9 / 36.8 / 33.8 / 42.1.
+// Chunking of the split-S decode attention, in multiples of the page, within
+// the LDS of the packed p (G * chunk * 4 bytes <= 48 KiB) and SPLIT_MAX_CHUNK.
+//
+// Below 256 (row, kv head) pairs: chunks of 256 to 1024 slots, cut until the
+// launch has about 256 blocks (one per CU: a CU draws no more than about 32
+// bytes per ns, so fewer leave bandwidth unused, and every chunk block sums
+// the whole row's denominator, so more cost more); for that reason no more
+// than 16 chunks per row either, where the limits above allow it. us per call,
+// 16 / 8 heads, at 256 / 512 / 1024 / 2048 slots per chunk: 1 x 4000 16.1 /
+// 17.7 / 22.3 / 32.2, 8 x 4000 29.1 / 25.9 / 25.7 / 35.0, 2 x 16384 48.9 /
+// 36.8 / 33.8 / 42.1.
+//
+// From 256 pairs on the pairs fill the chip by themselves, and scores and
+// partials through HBM only cost: as few chunks as the limits allow, of even
+// length, and where that is one (4096 slots at 1 or 2 query heads per kv head)
+// the one-block kernel takes the row. us per decode step of 4 layers, 16 / 8
+// heads, one block / chunks of 1024 / 2048 / 4096: 32 x 4000 460 / 509 / 518 /
+// -, 64 x 4000 672 / 788 / 754 / -, 128 x 4000 1135 / 1305 / 1267 / -, 32 x
+// 8100 855 / 783 / 726 / 741, 64 x 8100 1376 / 1287 / 1207 / 1176, 128 x 8100
+// 2549 / 2302 / 2188 / 2140 (24 rows, 192 pairs: 4000 431 / 457 / 493 / -,
+// 8100 819 / 666 / 625 / 692). us per call, 32 / 8 heads, one block / 1024 /
+// 2048: 64 x 4096 160 / 148 / 135, 128 x 4096 336 / 279 / 263; at 2048 slots
+// one block against two chunks 37 / 39 (32 rows), 47 / 63 (64), 100 / 135 (128).
 int detllm_attn_split_plan(int B, int S, int n_q, int n_kv, int* chunk, int* nsplit) {
   if (!chunk || !nsplit || B <= 0 || S <= 0 || n_q <= 0 || n_kv <= 0 || n_q % n_kv) return DI_EINVAL;
   const int G = n_q / n_kv;
   if (G > MAXG) return DI_ENOSYS;
+  const i64 cmax = imin(DECODE_LDS_BYTES / (4 * G) / DI_PAGE * DI_PAGE, SPLIT_MAX_CHUNK);
   const i64 blocks = (i64)B * n_kv;
-  const i64 want = blocks >= 256 ? 1 : (256 + blocks - 1) / blocks;
-  i64 ch = imin(((i64)S + want - 1) / want, 1024);
-  ch = imax(ch, ((i64)S + 15) / 16);
+  i64 ch;
+  if (blocks >= 256) {
+    const i64 ns = ((i64)S + cmax - 1) / cmax;
+    ch = ((i64)S + ns - 1) / ns;
+  } else {
+    const i64 want = (256 + blocks - 1) / blocks;
+    ch = imin(((i64)S + want - 1) / want, 1024);
+    ch = imax(ch, ((i64)S + 15) / 16);
+  }
   ch = (ch + DI_PAGE - 1) / DI_PAGE * DI_PAGE;
-  i64 cmax = DECODE_LDS_BYTES / (4 * G) / DI_PAGE * DI_PAGE;
-  if (cmax > SPLIT_MAX_CHUNK) cmax = SPLIT_MAX_CHUNK;
   ch = imax(imin(ch, cmax), (i64)2 * DI_PAGE);
   *chunk = (int)ch;
   *nsplit = (int)(((i64)S + ch - 1) / ch);

@@ -368,9 +368,12 @@ int detllm_attn_decode_split_sum(const int8_t* q8, const int64_t* tpos, const in
                                  int32_t* scores, int32_t* cmax, int64_t* out, int32_t* err,
                                  hipStream_t s);
 
-/* The chunking detllm_attn_decode_split is tuned for at (B, S, n_q, n_kv):
- * about 256 blocks, chunks of 256 to 1024 slots (more for rows past 16384, at
- * most 16 chunks up to 4096 slots each). Writes *chunk, *nsplit. */
+/* The chunking detllm_attn_decode_split is tuned for at (B, S, n_q, n_kv).
+ * Below 256 (row, kv head) pairs about 256 blocks: chunks of 256 to 1024 slots,
+ * at most 16 per row where the longest chunk allows it; from 256 pairs on as
+ * few chunks as it allows. The longest chunk is 4096 slots, less above 2 query
+ * heads per kv head (3072 at 4, 1536 at 8). *nsplit of 1: detllm_attn_decode
+ * (or detllm_qkv_attn_decode) is the faster call. Writes *chunk, *nsplit. */
 int detllm_attn_split_plan(int B, int S, int n_q, int n_kv, int* chunk, int* nsplit);
 
 /* Per-step bookkeeping of the graph-captured decode (src/detllm/graphed.py:

@@ -735,3 +735,31 @@ def test_attn_decode_op_routes(S, B, n_q, n_kv):
     call("detllm_attn_decode", q8, tpos, kp, vp, table, w, valid.view(torch.uint8), w * 128, B, S,
          n_q, n_kv, None, scratch, want, err)
     assert torch.equal(got, want) and int(err) == 0
+
+
+@pytest.mark.parametrize("B,n_q,n_kv,S", [(32, 16, 8, 4096), (32, 16, 8, 4097), (33, 16, 8, 4300),
+                                          (128, 2, 2, 8193), (64, 32, 8, 3100), (256, 8, 1, 1600)])
+def test_split_plan_of_many_pairs(B, n_q, n_kv, S):
+    """Rows of 256 and more (row, kv head) pairs at the planned chunking (one
+    chunk up to the longest, even ones past it) sum to the one-block kernel's
+    context."""
+    from idempotent_llm_amd._lib import attn_split_plan, call
+    print(f"[split plan of many pairs B={B} n_q={n_q} n_kv={n_kv} S={S}]", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(S)
+    w = -(-S // 128)
+    i8 = lambda *s: torch.randint(-128, 128, s, dtype=torch.int8, device="cuda", generator=g)
+    kp, vp = i8(B * w, n_kv, 128, 128), i8(B * w, n_kv, 128, 128)
+    table = torch.randperm(B * w, device="cuda", generator=g).to(torch.int32).view(B, w)
+    valid = torch.rand(B, w * 128, device="cuda", generator=g) < 0.8
+    valid[1, :S] = False
+    valid[2, :S - 1] = False
+    q8 = i8(B, n_q, 128)
+    tpos = torch.randint(1, 1 << 16, (B, n_q), device="cuda", generator=g)
+    chunk, ns = attn_split_plan(B, S, n_q, n_kv)
+    out = _split(q8, tpos, kp, vp, table, w, valid, B, S, n_q, n_kv, chunk)
+    assert out.shape[0] == ns
+    want = torch.full((B, n_q * 128), -7, dtype=I64, device="cuda")
+    scratch = torch.empty(B, n_q, (S + 15) // 16 * 16, dtype=torch.int32, device="cuda")
+    call("detllm_attn_decode", q8, tpos, kp, vp, table, w, valid.view(torch.uint8), w * 128, B, S,
+         n_q, n_kv, None, scratch, want, None)
+    assert torch.equal(out.sum(0), want)

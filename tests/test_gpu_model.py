@@ -379,3 +379,31 @@ def test_logits_digest_matches_host_formula(case):
     for r, g in zip(rows.cpu().numpy(), got):
         want = sum(mix((i << 32) | (int(x) & 0xFFFFFFFF)) for i, x in enumerate(r)) & M
         assert g & M == want
+
+
+def test_split_attention_of_many_rows(case, monkeypatch):
+    """One decode step of 128 rows (256 (row, kv head) pairs) past the longest
+    chunk: through the split-S attention in two chunks, and through the
+    one-block kernel, the same logits; one slot less than the longest chunk
+    stays whole."""
+    rec, m, _ = case
+    if rec["dims"]["hidden"] != 256:
+        pytest.skip("tiny model only (memory)")
+    import idempotent_llm_amd.model as mdl
+    from idempotent_llm_amd.model import KVCache
+    B, n, step = 128, 4100, 410
+    g = torch.Generator(device="cuda").manual_seed(5)
+    ids = torch.randint(0, m.vocab, (B, n + 1), device="cuda", generator=g)
+    pos = (torch.arange(n + 1, device="cuda") % 1000).expand(B, n + 1)
+    valid = torch.rand(B, n + 1, device="cuda", generator=g) < 0.9
+    valid[:, n] = True
+    assert m._split_plan(B, 4096) is None and m._split_plan(B, n + 1)[1] == 2
+    cache, runs = KVCache(), []
+    rows = torch.zeros(B, dtype=I64, device="cuda")
+    for lo in range(0, n, step):
+        m._forward(ids[:, lo:lo + step], pos[:, lo:lo + step], cache, valid[:, lo:lo + step], rows)
+    for thr in (mdl.SPLIT_MIN_SLOTS, 1 << 30):
+        monkeypatch.setattr(mdl, "SPLIT_MIN_SLOTS", thr)
+        cache.length = n
+        runs.append(m.forward(ids[:, n:], pos[:, n:], cache, valid[:, n:])[0])
+    assert torch.equal(runs[0], runs[1])

@@ -131,3 +131,24 @@ def test_missing_library_fails_loudly(monkeypatch, tmp_path):
         _lib.gemv_plan(8, 1024, 1024)
     with pytest.raises(_lib.LibraryMissing):
         _lib.call("detllm_igemv_plan", 8, 1024, 1024)
+
+
+@pytest.mark.skipif(not os.path.exists(LIB), reason="library not built (run build())")
+@pytest.mark.parametrize("n_q,n_kv", [(8, 8), (16, 8), (32, 8), (64, 8), (8, 1), (4, 2)])
+def test_attn_split_plan_host_entry(n_q, n_kv):
+    """Every plan is one the split launch takes, of chunks that cover the
+    slots. From 256 (row, kv head) pairs on a row is cut no further than the
+    longest chunk makes necessary: rows within it stay whole (the one-block
+    kernel), longer ones are cut evenly."""
+    from idempotent_llm_amd._lib import attn_split_plan
+    G = n_q // n_kv
+    longest = min(48 * 1024 // (4 * G) // 128 * 128, 4096)
+    for B in (1, 2, 7, 31, 32, 33, 64, 127, 128, 200, 256, 1000):
+        for S in (1, 127, 128, 129, 255, 256, 257, 1000, 1536, 1537, 2048, 2049, 3072, 3073,
+                  4000, 4096, 4097, 6144, 8192, 8193, 16384, 40000, 131071):
+            chunk, ns = attn_split_plan(B, S, n_q, n_kv)
+            assert chunk % 128 == 0 and 256 <= chunk <= longest, (B, S, chunk)
+            assert ns == -(-S // chunk), (B, S, chunk, ns)
+            if B * n_kv >= 256:
+                assert ns == -(-S // longest), (B, S, chunk, ns)
+                assert ns == 1 or chunk - S / ns < 128, (B, S, chunk, ns)
