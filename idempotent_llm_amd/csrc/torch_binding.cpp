@@ -411,6 +411,27 @@ Tensor op_attn_prefill(const Tensor& q8, const Tensor& tpos, const Tensor& kpool
   return out;
 }
 
+// Slots from which attn_decode cuts a row into chunks, G query heads per kv
+// head. A block per (row, kv head) leaves CUs idle when pairs are few; a chunk
+// block sums its row's whole denominator for each of its heads, so more heads
+// need longer rows, and more pairs (whose blocks fill the chip) longer ones
+// still. us per call, one block / chunks:
+//   pairs <= 64, G = 2: 768 slots 13.5 / 12.3, 1024 16.5 / 12.4, 4096 56 / 24;
+//     G = 4: 768 16.0 / 17.3, 896 18.2 / 17.7, 1024 19.1 / 17.7
+//   65 to 128 pairs, G = 2: 768 13.5 / 14.5, 1024 16.4 / 16.6, 1152 19 / 18.5,
+//     1280 20.4 / 18.2; G = 4: 1152 22 / 25, 1408 27 / 27, 1536 28 / 28
+//   G = 8: 768 19 / 27, 1536 30 / 31; from 1537 slots on the one block's scores
+//     (32 bytes a slot) are past its 48 KiB of LDS: 40 / 33
+// More than 128 pairs take one block at any length. At G = 2 that is the better
+// form to about 2048 slots only: 192 pairs 1024 slots 18.8 / 21.9, 2048 32 / 30,
+// 4096 58 / 42; 256 pairs 19.2 / 23.2, 32.5 / 32.5, 60 / 54.
+int64_t split_from(int64_t G, int64_t pairs) {
+  if (pairs > 128) return INT64_MAX;
+  if (G > 4) return 1537;
+  if (G > 2) return pairs <= 64 ? 896 : 1536;
+  return pairs <= 64 ? 768 : 1152;
+}
+
 Tensor op_attn_decode(const Tensor& q8, const Tensor& tpos, const Tensor& kpool,
                       const Tensor& vpool, const Tensor& table, const Tensor& valid, int64_t S,
                       const Tensor& err) {
@@ -419,11 +440,7 @@ Tensor op_attn_decode(const Tensor& q8, const Tensor& tpos, const Tensor& kpool,
   const int64_t G = n_q / n_kv;
   Tensor out = empty({B, n_q * 128}, at::kLong, q8);
   const Tensor qc = q8.contiguous(), tc = tpos.contiguous(), v = valid.view(at::kByte);
-  // Long rows of few (row, kv head) pairs: a block per pair leaves most CUs
-  // idle, so the rows are cut into chunks. us per call, one block / chunks:
-  // 1 x 1024 slots 17.6 / 13.6, 8 x 1024 19.4 / 15.3, 8 x 4096 58.2 / 26; at
-  // 576 slots, and from 32 rows on, the two are even.
-  if (B > 0 && S >= 768 && B * n_kv <= 128) {
+  if (B > 0 && S >= split_from(G, B * n_kv)) {
     int chunk = 0, ns = 0;
     check(detllm_attn_split_plan((int)B, (int)S, (int)n_q, (int)n_kv, &chunk, &ns),
           "detllm_attn_split_plan");

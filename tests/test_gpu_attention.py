@@ -763,3 +763,38 @@ def test_split_plan_of_many_pairs(B, n_q, n_kv, S):
     call("detllm_attn_decode", q8, tpos, kp, vp, table, w, valid.view(torch.uint8), w * 128, B, S,
          n_q, n_kv, None, scratch, want, None)
     assert torch.equal(out.sum(0), want)
+
+
+# (rows, query heads, kv heads, slots, whether the operator cuts the rows):
+# both sides of its rule at 64 and at 128 (row, kv head) pairs, 1, 2, 4 and 8
+# query heads per kv head
+OP_ROUTES = [(2, 4, 2, 1, False), (2, 4, 2, 767, False), (2, 4, 2, 768, True),
+             (32, 4, 2, 768, True), (33, 4, 2, 1151, False), (33, 4, 2, 1152, True),
+             (64, 2, 2, 1152, True), (65, 2, 2, 1152, False), (2, 2, 2, 768, True),
+             (2, 8, 2, 895, False), (2, 8, 2, 896, True), (33, 8, 2, 1535, False),
+             (33, 8, 2, 1536, True), (3, 8, 1, 1536, False), (3, 8, 1, 1537, True),
+             (129, 2, 1, 1300, False)]
+
+
+@pytest.mark.parametrize("B,n_q,n_kv,S,cut", OP_ROUTES)
+def test_attn_decode_op_vs_oracle(B, n_q, n_kv, S, cut):
+    """The registered decode attention against the oracle on both sides of
+    its chunking rule; the route shows in its allocations (out, and scores
+    and chunk maxima or the one block's scratch)."""
+    from idempotent_llm_amd import torch_ops  # noqa: F401
+    print(f"[attn_decode op vs oracle B={B} n_q={n_q} n_kv={n_kv} S={S}]", flush=True)
+    cap = -(-S // 128) * 128
+    q8, kc, vc, valid, sm, sk, tpos = _prefill_case(B, n_q, n_kv, 1, S - 1, cap, S + B, 29, 34,
+                                                    dead_prefix=S // 2)
+    want = _prefill_oracle(q8, kc, vc, valid, sm, sk, S - 1)[:, 0]
+    d = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()
+    kp, vp, table, width, vmask = paged(kc, vc, valid, seed=B)
+    q, t = d(q8[:, :, 0]), d(tpos[:, :, 0, 0])
+    err = torch.zeros(1, dtype=torch.int32, device="cuda")
+    before = torch.cuda.memory_stats()["allocation.all.allocated"]
+    out = torch.ops.detllm_rocm.attn_decode(q, t, kp, vp, table, vmask, S, err)
+    made = torch.cuda.memory_stats()["allocation.all.allocated"] - before
+    scratch = n_q // n_kv * (-(-S // 16) * 16) * 4 > 48 * 1024
+    assert np.array_equal(out.cpu().numpy(), want)
+    assert made == (3 if cut else 2 if scratch else 1)
+    assert int(err) == 0
