@@ -9,6 +9,8 @@
 // scale and DI-Exp constant).
 #pragma once
 
+#include <type_traits>
+
 #include "common.h"
 
 namespace di {
@@ -617,11 +619,14 @@ namespace di {
 // entries load while the current row computes, the Q rows' DI-Exp constants
 // (one lane's serial chain) come from NG lanes side by side at the end, and a
 // lane's NG consecutive slots of V go out as one word instead of NG bytes.
-// Measured at 2048 rows of 32 heads (32 MB of product): 35.5 -> 26.0 us, vector
-// instructions 14.3 M -> 11.0 M (70 % of the issue slots), 4096 rows 64.2 ->
-// 44.7 us. The kinds are separate code (qkv_rows_kind), and rows outside the
-// fp64 forms' bounds are redone after the passes: either one inside the
-// passes costs enough registers to halve the waves in flight.
+// Measured at 2048 rows of 32 heads (32 MB of product), one row against four
+// rows per lane: launched back to back 34.8 -> 25.0 us (in a prefill's trace,
+// its inputs fresh from the product, 29), vector instructions 14.3 M -> 11.0 M
+// (70 % of the issue slots), 4096 rows 63 -> 43 us. The kinds are separate code
+// (qkv_rows_kind), and rows outside the fp64 forms' bounds are redone after the
+// passes: either one inside the passes costs enough registers to halve the
+// waves in flight. Four waves per SIMD still take spills at NG = 4 (68 vector
+// registers of 128, outside the inner chains) and a few at NG = 1 (6).
 // Same arithmetic and the same integers as qkv_head.
 typedef short v4s_u __attribute__((ext_vector_type(4), aligned(2)));  // any int16 alignment
 
@@ -649,7 +654,7 @@ __device__ __forceinline__ void qkv_rows_redo(const QKVArgs& a, int R, int r0, i
 // row left the fp64 forms' bounds: what they stored is redone (qkv_rows_redo).
 template <int NG, int KIND>
 __device__ __forceinline__ uint32_t qkv_rows_kind(const QKVArgs& a, int R, int r0, int slotw) {
-  static_assert(NG == 1 || NG == 4, "rows per lane");
+  static_assert(NG == 1 || NG == 2 || NG == 4, "rows per lane");
   const int lane = threadIdx.x & 63, g = lane >> 4, j = lane & 15;
   const int n_heads = a.n_q + 2 * a.n_kv;
   const int group = a.n_q / a.n_kv;
@@ -747,17 +752,18 @@ __device__ __forceinline__ uint32_t qkv_rows_kind(const QKVArgs& a, int R, int r
         p[k] = pn[k];
       }
     }
-    // the lane's NG slots: one word when they are NG consecutive slots of one
+    // the lane's NG slots: one store when they are NG consecutive slots of one
     // row that start at a multiple of NG (then they share a page too), else
     // a byte each
+    using VWord = std::conditional_t<NG == 4, uint32_t, uint16_t>;
     const int b0 = row(0) / a.T;
     i64 slot;
     const int pg = place(0, &slot);
-    if (NG == 4 && rl + NG <= R && (rl + NG - 1) / a.T == b0 && (slot & (NG - 1)) == 0) {
+    if (NG > 1 && rl + NG <= R && (rl + NG - 1) / a.T == b0 && (slot & (NG - 1)) == 0) {
       if (pg >= 0) {
 #pragma unroll
         for (int k = 0; k < 8; ++k)
-          *(uint32_t*)(a.kv.vchan(pg, kvh, c[k]) + (slot & (DI_PAGE - 1))) = word[k];
+          *(VWord*)(a.kv.vchan(pg, kvh, c[k]) + (slot & (DI_PAGE - 1))) = (VWord)word[k];
       }
     } else {
 #pragma unroll 1
@@ -904,13 +910,27 @@ __device__ __forceinline__ uint32_t qkv_rows_kind(const QKVArgs& a, int R, int r
   return bad;
 }
 
+// a: the kernel's first argument (the redo reads it again from the argument
+// segment, so that the passes do not hold all of it in scalar registers:
+// three to four waves per SIMD at NG = 1, 2048 rows of 48 heads at NG = 4 36.2
+// -> 35.3 us).
 template <int NG>
 __device__ __forceinline__ void qkv_rows(const QKVArgs& a, int R, int r0, int slotw) {
   uint32_t bad;
   if (slotw < a.n_q) bad = qkv_rows_kind<NG, 0>(a, R, r0, slotw);
   else if (slotw < a.n_q + a.n_kv) bad = qkv_rows_kind<NG, 1>(a, R, r0, slotw);
   else bad = qkv_rows_kind<NG, 2>(a, R, r0, slotw);
-  if (DI_UNLIKELY(bad != 0)) qkv_rows_redo<NG>(a, R, r0, slotw, bad);
+  if (DI_UNLIKELY(bad != 0)) {
+    struct Words {
+      u64 w[sizeof(QKVArgs) / 8];
+    } args;
+    static_assert(sizeof(QKVArgs) % 8 == 0 && std::is_trivially_copyable_v<QKVArgs>);
+    auto src = (const __attribute__((address_space(4))) u64*)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(src));  // (not the loads made at the kernel's start)
+#pragma unroll
+    for (int i = 0; i < (int)(sizeof(QKVArgs) / 8); ++i) args.w[i] = src[i];
+    qkv_rows_redo<NG>(__builtin_bit_cast(QKVArgs, args), R, r0, slotw, bad);
+  }
 }
 
 }  // namespace di

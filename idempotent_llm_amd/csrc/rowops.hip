@@ -1119,11 +1119,11 @@ __global__ __launch_bounds__(RT) void k_qkv_epilogue(QKVArgs a) {
 }
 
 // Many token rows (prefill): one wave per (head slot, 4 NG rows), head-major
-// so a block's waves share a head's scale vectors. Registers: at NG = 4 a
-// wave lives for four passes, and four waves per SIMD (128 VGPRs) keep the
-// vector unit busy; at NG = 1 three waves without spills beat four with them.
+// so a block's waves share a head's scale vectors. Waves per SIMD: four, at NG
+// = 2 three (149 VGPRs; four spill 72: 1000 rows of 32 heads 17.9 against 16.9
+// us, 500 13.8 against 10.7).
 template <int NG>
-__global__ __launch_bounds__(RT, NG == 4 ? 4 : 3) void k_qkv_epilogue_rows(QKVArgs a, int R,
+__global__ __launch_bounds__(RT, NG == 2 ? 3 : 4) void k_qkv_epilogue_rows(QKVArgs a, int R,
                                                                            int ngroups) {
   keep_hidden_args();
   const int heads = a.n_q + 2 * a.n_kv;
@@ -2233,19 +2233,24 @@ int detllm_qkv_epilogue(const int32_t* P, int nsplit, int64_t split_stride, int 
   const int R = B * T;
   // the rows layout reads P 16 bytes at a time
   if (R > 64 && (nsplit == 1 || split_stride % 4 == 0) && ((uintptr_t)P & 15) == 0) {
-    // Rows per lane: four once the launch has about a round of waves left at
-    // four rows per lane (36864 (row, head) pairs, 1152 rows of 32 heads: two
-    // waves per SIMD), where sharing the scale vectors pays; below, one row
-    // per lane and four times the waves. Measured at 32 heads, four against
-    // one: 200 rows 14.9 / 7.7 us, 1024 rows 18.9 / 18.3, 1200 rows 20.9 /
-    // 22.7, 2048 rows 26.0 / 35.4.
-    const bool many = (i64)R * heads >= 36864;
-    const int rows = many ? 16 : 4;
-    const int ngroups = (R + rows - 1) / rows;
+    // Rows per lane, by (row, head) pairs: a lane that takes more rows shares
+    // the scale vectors among them, one that takes fewer leaves more waves to
+    // the chip. One row up to 21504 pairs (a round and a third of four waves
+    // per SIMD), two up to 49152 (two rounds of three), then four. us at 1 / 2
+    // / 4 rows per lane: 32 heads 200 rows 7.2 / 7.6 / 14.1, 600 11.5 / 12.9 /
+    // 14.5, 700 13.8 / 13.1 / 17.9, 1000 18.6 / 16.9 / 18.6, 1200 - / 20.2 /
+    // 20.1, 1500 - / 23.1 / 23.5, 2048 - / 27.9 / 25.0; 10 heads 2048 rows 11.9
+    // / 12.2 / 17.7, 3000 17.2 / 16.7 / 19.2, 4096 - / 18.6 / 22.7; 48 heads 400
+    // rows 11.4 / 11.5 / 14.5, 500 14.0 / 12.8 / 18.0, 1000 - / 22.2 / 23.3, 1152
+    // - / 25.3 / 24.0.
+    const i64 pairs = (i64)R * heads;
+    const int ng = pairs < 21504 ? 1 : (pairs < 49152 ? 2 : 4);
+    const int ngroups = (R + 4 * ng - 1) / (4 * ng);
     const i64 waves = (i64)ngroups * heads;
     if (waves > 0x7fffffff) return DI_ERANGE;
     const dim3 grid((unsigned)((waves + 3) / 4));
-    if (many) hipLaunchKernelGGL(k_qkv_epilogue_rows<4>, grid, dim3(RT), 0, s, a, R, ngroups);
+    if (ng == 4) hipLaunchKernelGGL(k_qkv_epilogue_rows<4>, grid, dim3(RT), 0, s, a, R, ngroups);
+    else if (ng == 2) hipLaunchKernelGGL(k_qkv_epilogue_rows<2>, grid, dim3(RT), 0, s, a, R, ngroups);
     else hipLaunchKernelGGL(k_qkv_epilogue_rows<1>, grid, dim3(RT), 0, s, a, R, ngroups);
   } else {
     hipLaunchKernelGGL(k_qkv_epilogue, dim3(R, (heads + 3) / 4), dim3(RT), 0, s, a);

@@ -608,20 +608,13 @@ def test_qkv_epilogue_every_path(variant, B, T):
         np.testing.assert_array_equal(v[:, :, slot].cpu().numpy(), want_v[:, :, 0])
 
 
-@pytest.mark.parametrize("variant", ["none", "ranges", "gamma"])
-@pytest.mark.parametrize("B,T,slot", [(3, 401, 0), (2, 640, 128), (5, 256, 3), (1, 1153, 126)])
-def test_qkv_epilogue_rows_per_lane(variant, B, T, slot):
-    """The epilogue of many rows (four rows per lane) against the oracle: a
-    last group of fewer rows, groups that cross a batch row or a page, V slots
-    that start inside a word, and heads and rows that leave the fp64 forms
-    (_plant's channels, a zero head, a row whose V numerators wrap)."""
+def _rows_per_lane(variant, B, T, slot):
     from idempotent_llm_amd._lib import call
     print(f"[qkv epilogue rows per lane {variant} B={B} T={T} slot={slot}]", flush=True)
     dims = art.MID
     nq, nkv, hd = dims["n_q_heads"], dims["n_kv_heads"], 128
     prm = _plant(_layer_params(dims, 6), variant, nq, nkv)
     R = B * T
-    assert R * (nq + 2 * nkv) >= 36864
     rnd = torch.Generator().manual_seed(B * 1000 + T)
     P = torch.randint(-(1 << 19), 1 << 19, (1, R, (nq + 2 * nkv) * hd), generator=rnd,
                       dtype=torch.int32)
@@ -656,6 +649,17 @@ def test_qkv_epilogue_rows_per_lane(variant, B, T, slot):
         np.testing.assert_array_equal(v[:, :, slot:].cpu().numpy(), want_v)
         assert torch.equal(k[:, :, :slot].cpu(), k0[:, :, :slot])   # earlier slots untouched
         assert torch.equal(v[:, :, :slot].cpu(), v0.transpose(2, 3)[:, :, :slot])
+
+
+@pytest.mark.parametrize("variant", ["none", "ranges", "gamma"])
+@pytest.mark.parametrize("B,T,slot", [(3, 401, 0), (2, 640, 128), (5, 256, 3), (1, 1153, 126)])
+def test_qkv_epilogue_rows_per_lane(variant, B, T, slot):
+    """The epilogue of many rows (two rows per lane) against the oracle: a
+    last group of fewer rows, groups that cross a batch row or a page, V slots
+    that start inside a word, and heads and rows that leave the fp64 forms
+    (_plant's channels, a zero head, a row whose V numerators wrap)."""
+    assert B * T * (art.MID["n_q_heads"] + 2 * art.MID["n_kv_heads"]) >= 36864
+    _rows_per_lane(variant, B, T, slot)
 
 
 @pytest.mark.parametrize("T,S_past", [(128, 0), (1, 128), (129, 0), (100, 156), (257, 0),
@@ -798,3 +802,13 @@ def test_attn_decode_op_vs_oracle(B, n_q, n_kv, S, cut):
     assert np.array_equal(out.cpu().numpy(), want)
     assert made == (3 if cut else 2 if scratch else 1)
     assert int(err) == 0
+
+
+@pytest.mark.parametrize("variant", ["none", "ranges", "gamma"])
+@pytest.mark.parametrize("B,T,slot", [(3, 224, 1), (1, 1535, 0), (1, 1536, 126), (4, 401, 0),
+                                      (7, 256, 3)])
+def test_qkv_epilogue_rows_per_lane_lines(variant, B, T, slot):
+    """The same on both sides of the line to four rows per lane (49152 (row,
+    head) pairs: 1536 rows of 32 heads) and on the line to two (21504: 672
+    rows); the sizes above take two."""
+    _rows_per_lane(variant, B, T, slot)
