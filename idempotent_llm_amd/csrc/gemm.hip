@@ -890,19 +890,27 @@ int detllm_igemm_nt(const int8_t* A, const int8_t* B, int32_t* C, int M, int N, 
   // kernels); their direct-to-LDS loads need 16-byte operands, k_gemm_nt's do not
   const bool aligned = (((uintptr_t)A | (uintptr_t)B | (uintptr_t)sA | (uintptr_t)sB) & 15) == 0;
   if (K % G2_BK == 0 && (M > 64 || aligned)) {
-    // Tile shape by tile count, from sweeps of every shape over the model's
-    // four products at 65 to 2048 rows. n = tiles of 128 x 64; us of the taken
-    // shape against 128 x 64 (one block per CU):
-    //   n <= 64: 64 x 32 in four K groups, four times the blocks (o and down
-    //     at 65 to 512 rows: 6.2 / 8.2 and 7.5 / 10.7)
+    // Tile shape by tile count, from sweeps over the model's four products at
+    // 65 to 2048 rows and over ragged shapes (N from 1030 to 6151, K from 128 to
+    // 3072). n = tiles of 128 x 64; us of the taken shape against 128 x 64 (one
+    // block per CU), the general one:
+    //   n <= 64, K >= 768: 64 x 32 in four K groups, four times the blocks (o and
+    //     down at 65 to 512 rows: 6.2 / 8.2 and 7.5 / 10.7). Shorter K: 64 x 64
+    //     without groups (512 x 1024, K = 256: 3.5 / 3.7, groups 4.1; K = 640:
+    //     4.4 / 4.7, groups 4.5)
     //   n <= 128, K >= 2048: 64 x 64 in two K groups (1024 rows: 7.9 / 9.0 and
     //     9.9 / 11.7); shorter K: 64 x 64 without groups (gate|up at 100 rows
     //     6.1 / 6.6; in groups 6.3: four steps each, and the sum costs as much)
     //   n <= 256: 128 x 64
-    //   n <= 512: 64 x 128, two blocks per CU (q|k|v at 1024 rows 9.7 / 11.5)
-    //   more: 128 x 128, two per CU (gate|up at 1024 rows 12.6 / 15.7), and by
-    //     their own counts 128 x 192 (two per CU) where it divides N (gate|up
-    //     at 2048 rows) and 256 x 256 for large products.
+    //   n <= 512: 64 x 128, two blocks per CU, where that is one round and pays
+    //     (narrow_pays below; q|k|v at 1024 rows 9.7 / 11.5)
+    //   more: 128 x 128, two per CU, where N is whole 64-byte lines of C (gate|up
+    //     at 1024 rows 12.6 / 15.7): its two 32-column runs per row are written
+    //     apart, so a line they share goes out twice (1501 x 4001, K = 256 13.1 /
+    //     10.6). Long K hides the stores: 12.9 / 14.3 at N % 8 = 0, K = 640; K of
+    //     2048 0.88 of 128 x 64 at odd N, of 1024 1.05
+    //   and by their own counts 256 x 256 for large products, 128 x 192 (two per
+    //     CU) where it divides N (gate|up at 2048 rows) and 128 x 128.
     auto tiles = [&](int bm, int bn) { return (i64)((M + bm - 1) / bm) * ((N + bn - 1) / bn) * batch; };
 #define DI_GEMM2(BM, BN, S, WGM, WGN, MINB, KG)                                                 \
   do {                                                                                          \
@@ -913,12 +921,26 @@ int detllm_igemm_nt(const int8_t* A, const int8_t* B, int32_t* C, int M, int N, 
                        (i64)sC, tm_, tn_);                                                      \
   } while (0)
     const i64 n = tiles(128, 64);
+    const bool lines = N % 16 == 0;  // rows of C start on 64-byte lines
+    const bool square_pays = lines || K >= (N % 8 == 0 ? 640 : 1536);
+    // 64 x 128 for 256 < n <= 512. A second round of few blocks costs as much as
+    // the first (3712 x 1056, 522 tiles, K = 512: 9.1 / 7.5). From K = 1024 on B
+    // is what is read, twice as often as by 128 rows, unless each XCD keeps its
+    // own columns (tile columns in fours) or they are few against the rows: 512 x
+    // 4128, K = 3072 24.2 / 20.9 and 896 x 3080 24.4 / 22.0, but 512 x 5000 0.81
+    // and 1118 x 3264, K = 2176 15.5 / 18.9. At N off the lines the two blocks of a CU also share lines of
+    // C: up to 320 tiles (360 at N % 4 = 0; 1408 x 1500, K = 256 0.78, but 1280 x
+    // 3113, 500 tiles 10.3 / 8.3), with longer K up to 400, from 2048 on all.
+    const i64 tm = (M + 63) / 64, tn = (N + 127) / 128, narrow = tm * tn * batch;
+    const i64 ragged_max = K >= 2048 ? 512 : (K >= 1024 ? 400 : (N % 4 == 0 ? 360 : 320));
+    const bool narrow_pays = narrow <= (lines ? 512 : ragged_max) &&
+                             (K < 1024 || tn % 4 == 0 || (K < 2560 ? 2 * tm : tm) >= tn);
     if (tiles(256, 256) >= 448) DI_GEMM2(256, 256, 2, 4, 2, 1, 1);
     else if (N % 192 == 0 && tiles(128, 192) >= 448) DI_GEMM2(128, 192, 2, 2, 2, 2, 1);
-    else if (n > 512) DI_GEMM2(128, 128, 2, 2, 2, 2, 1);
-    else if (n > 256) DI_GEMM2(64, 128, 3, 2, 2, 2, 1);
+    else if (tiles(128, 128) >= 448 || (n > 512 && square_pays)) DI_GEMM2(128, 128, 2, 2, 2, 2, 1);
+    else if (n > 256 && n <= 512 && narrow_pays) DI_GEMM2(64, 128, 3, 2, 2, 2, 1);
     else if (n > 128) DI_GEMM2(128, 64, 4, 4, 2, 1, 1);
-    else if (n <= 64) DI_GEMM2(64, 32, 3, 2, 1, 1, 4);
+    else if (n <= 64 && K >= 768) DI_GEMM2(64, 32, 3, 2, 1, 1, 4);
     else if (K >= 2048) DI_GEMM2(64, 64, 4, 2, 2, 1, 2);
     else DI_GEMM2(64, 64, 4, 2, 2, 2, 1);
 #undef DI_GEMM2

@@ -143,3 +143,18 @@ def test_operators_refuse_other_ranks():
             f()
     with pytest.raises(ValueError):
         ops.attn_decode(i8[0, 0], v, i8[:, :0], i8, i32[0, 0, 0], i8[0, 0, 0].bool(), 1, i32)
+
+
+# the lines of the rules that follow K and the alignment of N: four K groups
+# from K = 768, 128 x 128 off whole lines of C, 64 x 128 by its tiles, the tile
+# columns and N
+LINE_CASES = [(512, 1024, 640), (512, 1024, 768), (1501, 4001, 256), (1501, 4001, 1536),
+              (1024, 4104, 512), (1024, 4104, 640), (1500, 4016, 128), (3712, 1056, 512),
+              (512, 4128, 896), (512, 4128, 1024), (512, 5000, 1024), (1118, 3264, 1152),
+              (1408, 1500, 256), (1280, 3113, 256), (1280, 3113, 2048), (900, 3080, 1024),
+              (2048, 1271, 1024)]
+
+
+@pytest.mark.parametrize("M,N,K", LINE_CASES)
+def test_tile_rule_lines(M, N, K):
+    test_tile_rules(M, N, K)
