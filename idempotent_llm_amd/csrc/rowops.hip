@@ -1888,26 +1888,28 @@ void launch_pro(const ProGemv& g, int ni, int ksplit, const ResNormArgs& ra, con
 
 // The wave-per-row launch of a prefill-sized residual / norm-quant call
 // (C = 512 or 1024 columns); false: the caller launches the block-per-row
-// kernel. A wave per row has no barriers, but its chain over 16 columns per
-// lane is long; up to 640 rows a block per row (four columns per lane) fits
-// the chip two or three blocks per CU and is done sooner: residual rows 320 /
-// 512 / 700 / 1024 / 2048 take 7.3 / 7.6 / 8.8 / 10.1 / 14.4 us as blocks, 8.6
-// / 8.8 / 9.1 / 9.3 / 12.5 as waves. (The norm-quant alone, a shorter chain,
-// takes the wave at every size: 512 rows 6.0 us.)
-constexpr int ROWS_WAVE_MIN = 641;
+// kernel. A wave per row has no barriers, but its chain over 16 (8) columns per
+// lane is long: a block per row (four columns per lane) is done sooner while
+// all its blocks run at once, three per CU at 1024 columns, and at 512 (half
+// the wave's chain) one per CU. us of residual rows as blocks / waves, one
+// partial: 1024 columns 200 rows 5.5 / 7.5, 500 6.6 / 7.7, 760 7.6 / 7.9, 800
+// 8.6 / 8.0, 1024 8.9 / 8.1; 512 columns 256 rows 5.4 / 5.6, 300 6.4 / 5.7, 640
+// 7.4 / 5.8 (four partials: 760 rows 8.0 / 8.4, 800 8.9 / 8.5; 256 5.5 / 5.8,
+// 300 6.6 / 5.9). The norm-quant alone, a shorter chain, takes the wave at
+// every size (1024 columns, 512 rows 5.3 us).
+static int residual_block_rows(int C) { return C == 1024 ? 768 : 256; }
 template <int MODE>
 static bool rows_wave_launch(int R, int C, hipStream_t s, ResNormArgs& a) {
-  if (R <= (MODE == 1 ? ROWS_WAVE_MIN - 1 : 64) || (C != 512 && C != 1024)) return false;
+  if ((C != 512 && C != 1024) || R <= (MODE == 1 ? residual_block_rows(C) : 64)) return false;
   a.nt = 64;
   const dim3 grid((unsigned)((R + 3) / 4));
   // (one partial: its loads alone; 2048 rows 12.4 -> 11.6 us, 4096 20.7 -> 19.4)
-  const bool one = MODE != 1 || a.nsplit == 1;
-  if (C == 1024) {
-    if (one) hipLaunchKernelGGL((k_residual_normq_w<16, MODE, 1>), grid, dim3(256), 0, s, a, R);
-    else hipLaunchKernelGGL((k_residual_normq_w<16, MODE, 4>), grid, dim3(256), 0, s, a, R);
+  if (MODE == 1 && a.nsplit > 1) {
+    if (C == 1024) hipLaunchKernelGGL((k_residual_normq_w<16, 1, 4>), grid, dim3(256), 0, s, a, R);
+    else hipLaunchKernelGGL((k_residual_normq_w<8, 1, 4>), grid, dim3(256), 0, s, a, R);
   } else {
-    if (one) hipLaunchKernelGGL((k_residual_normq_w<8, MODE, 1>), grid, dim3(256), 0, s, a, R);
-    else hipLaunchKernelGGL((k_residual_normq_w<8, MODE, 4>), grid, dim3(256), 0, s, a, R);
+    if (C == 1024) hipLaunchKernelGGL((k_residual_normq_w<16, MODE, 1>), grid, dim3(256), 0, s, a, R);
+    else hipLaunchKernelGGL((k_residual_normq_w<8, MODE, 1>), grid, dim3(256), 0, s, a, R);
   }
   return true;
 }

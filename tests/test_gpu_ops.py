@@ -496,6 +496,53 @@ def test_residual_normq_every_path(big_col):
     eq(Cg.sum(0), ogemm.int_gemm(want[2], w8.T))
 
 
+@pytest.mark.parametrize("ns", [1, 2, 5])
+@pytest.mark.parametrize("C", [512, 1000, 1024])
+@pytest.mark.parametrize("R", [65, 256, 257, 640, 768, 769, 1025])
+def test_residual_normq_row_layouts(R, C, ns):
+    """The rows of the two tests above (every renormalisation branch, every
+    fp64 and int64 path) at prefill sizes, on both sides of the lines between
+    a block and a wave per row and with one and several partials of the
+    product, against the oracle."""
+    from idempotent_llm_amd._lib import call
+    print(f"[residual_normq row layouts R={R} C={C} ns={ns}]", flush=True)
+    rng = np.random.default_rng(R + C + ns)
+    scale = [2 ** 29 - 3, 2 ** 20, 2 ** 28, 0, 0, 2 ** 27, 2 ** 12, 2 ** 29]
+    rows = [(40000, 1 << 20, None), (40000, 1 << 20, 58), (40000, 1 << 20, 70),
+            (3, 4, -25), (3, 4, -40), (3, 4, -60), (1 << 33, 1 << 20, None),
+            (-(1 << 31), 1 << 20, None)]
+    n = len(scale) + len(rows)
+    h = np.stack([rng.integers(-s, s + 1, C) if s else np.zeros(C, I64) for s in scale]
+                 + [rng.integers(-(1 << 26), 1 << 26, C) for _ in rows])
+    h[4, C // 3] = 5
+    P = np.stack([rng.integers(-(1 << 20), 1 << 20, C) for _ in scale]
+                 + [rng.integers(-p, p + 1, C) for _, p, _ in rows])
+    P[3] = P[4] = 0
+    col_m = rng.integers(1 << 15, 1 << 16, C).astype(I64)
+    col_m[C // 2] = -((1 << 21) - 1)
+    k_res = np.full(n, 24, I64)
+    row_m = np.array([*rng.integers(1 << 15, 1 << 16, len(scale)), *(m for m, _, _ in rows)], I64)
+    _, _, dk0 = ody.requant_i32_common(P, row_m[:, None], np.zeros((n, 1), I64), col_m, 20,
+                                       target_bits=20)
+    row_k = np.array([20, 24, 26, 20, 20, 30, 40, 19]
+                     + [20 if rel is None else 24 + rel - dk0[8 + i, 0]
+                        for i, (_, _, rel) in enumerate(rows)], I64)
+    sm_m = rng.integers(1 << 15, 1 << 16, C).astype(I64)
+    want = _normq_oracle(P.astype(np.int32), row_m, row_k, col_m, 20, h.astype(np.int32), k_res,
+                         sm_m, 15)
+    pick = np.concatenate([rng.permutation(n) for _ in range(-(-R // n))])[:R]
+    parts = rng.integers(-(1 << 20), 1 << 20, (ns, R, C))
+    parts[0] = P[pick] - parts[1:].sum(axis=0)
+    hg, kg = g(h[pick].astype(np.int32)), g(k_res[pick])
+    x8 = torch.empty(R, C, dtype=torch.int8, device="cuda")
+    xm = torch.empty(R, dtype=torch.int64, device="cuda")
+    xk = torch.empty(R, dtype=torch.int64, device="cuda")
+    call("detllm_residual_normq", g(parts.astype(np.int32)), ns, R * C, R, C, g(row_m[pick]),
+         g(row_k[pick]), g(col_m), 20, 20, hg, kg, g(sm_m), 15, x8, xm, xk, None, 0, 0, 0, 0)
+    for got, w in zip((hg, kg, x8, xm, xk), want):
+        eq(got, w[pick])
+
+
 def test_igemv_prefetch_variant_same_product():
     """detllm_igemv_nt_pf (skinny GEMM + prefetch hint) gives the product of
     detllm_igemv_nt, with 0-4 ranges of any multiple-of-4 size; bad ranges are
