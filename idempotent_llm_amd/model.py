@@ -95,15 +95,14 @@ class LayerWeights:
     # per-channel divisors of the static K requantisation, [n_kv * 128, 4]
     # int64 (detllm_kq_est): layer constants computed once at load
     kq_est: torch.Tensor | None = None
-    # the model's RoPE tables and their size (cos, sin, max_pos)
-    rope: tuple = ()
 
     @property
     def epi(self) -> tuple:
-        """The Q/K/V epilogue's layer constants in its argument order."""
+        """The Q/K/V epilogue's layer constants in its argument order (the
+        model's RoPE tables follow them)."""
         return (self.q_m, self.q_k, self.k_m, self.k_k, self.v_m, self.v_k, self.q_norm_m,
                 self.q_norm_k, self.k_norm_m, self.k_norm_k, self.qs_m, self.qs_k, self.kq_m,
-                self.kq_k, self.ks_m, self.ks_k, self.vq_m, self.vq_k, *self.rope)
+                self.kq_k, self.ks_m, self.ks_k, self.vq_m, self.vq_k)
 
     # the reference's field names (model.py:41-64) as views of the kernel
     # layout, for code written against the reference class (seam overrides)
@@ -256,7 +255,6 @@ class IntQwen3:
             L.pf_mlp = _pack(L, ["gate_m", "up_m", "ds_m"])
             L.kq_est = torch.empty(L.kq_m.numel(), 4, dtype=I64, device=dev)
             call("detllm_kq_est", L.kq_m, L.kq_k, L.kq_m.numel(), 20 + L.k_norm_k, L.kq_est)
-            L.rope = (self.rope_cos, self.rope_sin, self.max_pos)
         self._greedy_scratch = {}
         self._plans: dict = {}
         self._split_plans: dict = {}
@@ -514,7 +512,7 @@ class IntQwen3:
             q8 = ws.buf("q8", (B, nq, 1, hd), torch.int8)
             tpos = ws.buf("tpos", (B, nq, 1), I64)
             call("detllm_qkv_epilogue", P, ns, st, B, 1, nq, nkv, xm, xk, pos,
-                 *L.epi, q8, tpos, None,
+                 *L.epi, self.rope_cos, self.rope_sin, self.max_pos, q8, tpos, None,
                  *cache.layer_args(li), cache.len_idx if static else None,
                  0 if static else S_past, L.kq_est, self._err)
             scores = ws.buf("scores", (B, nq, nsp * chunk), torch.int32)
@@ -529,7 +527,7 @@ class IntQwen3:
             # decode: Q/K/V epilogue and attention in one launch
             scratch = self._decode_scratch(ws, B, S)
             args = (P, ns, st, B, nq, nkv, xm, xk, pos,
-                    *L.epi,
+                    *L.epi, self.rope_cos, self.rope_sin, self.max_pos,
                     *cache.layer_args(li), cache.len_idx if static else None,
                     0 if static else S_past, valid, cache.cap, S,
                     cache.nslots if static else None, scratch, attn, self._err)
@@ -626,7 +624,7 @@ class IntQwen3:
         q8 = ws.buf("q8", (B, nq, T, hd), torch.int8)
         tpos = ws.buf("tpos", (B, nq, T), I64)
         call("detllm_qkv_epilogue", P, ns, st, B, T, nq, nkv, xm, xk, pos,
-             *L.epi, q8, tpos, None,
+             *L.epi, self.rope_cos, self.rope_sin, self.max_pos, q8, tpos, None,
              *cache.layer_args(li), cache.len_idx if static else None,
              0 if static else S_past, L.kq_est, self._err)
         valid = ws.valid
@@ -653,7 +651,7 @@ class IntQwen3:
         tpos = torch.empty(B, nq, T, dtype=I64, device=dev)
         dbg = torch.empty(B, nq, T, 4, dtype=I64, device=dev)
         call("detllm_qkv_epilogue", P, ns, st, B, T, nq, nkv, xm, xk, pos,
-             *L.epi, q8, tpos, dbg,
+             *L.epi, self.rope_cos, self.rope_sin, self.max_pos, q8, tpos, dbg,
              *cache.layer_args(li), None, S_past, L.kq_est, self._err)
         qm, qk = dbg[..., 0:1], dbg[..., 1:2]
         Pfull = P.view(ns, B, T, -1).sum(dim=0, dtype=torch.int32) if ns > 1 else \

@@ -407,3 +407,32 @@ def test_split_attention_of_many_rows(case, monkeypatch):
         cache.length = n
         runs.append(m.forward(ids[:, n:], pos[:, n:], cache, valid[:, n:])[0])
     assert torch.equal(runs[0], runs[1])
+
+
+def test_rope_tables_are_the_models_own(case):
+    """Tables assigned to the model after the load are the ones every path
+    uses: shifted down by one position, they give the logits of positions one
+    lower, in prefill, eager decode and graphed decode."""
+    from idempotent_llm_amd.graphed import GraphedDecode
+    rec, m, _ = case
+    ids = _ids(rec)[None].repeat(2, 1)
+    T = ids.shape[1]
+    pos = torch.arange(T, device="cuda").expand(2, T)
+    runs, cos, sin = [], m.rope_cos, m.rope_sin
+    try:
+        for off in (0, 1):
+            m.rope_cos, m.rope_sin = cos.roll(off, 0), sin.roll(off, 0)
+            out = []
+            logits, _, _, cache = m.forward(ids, pos + off, None)
+            out.append(logits)
+            cur = m.greedy_pick(logits[:, -1])
+            logits, _, _, cache = m.forward(cur[:, None], pos[:, :1] + T + off, cache)
+            out.append(logits)
+            cur = m.greedy_pick(logits[:, -1])
+            gd = GraphedDecode(m, cache, torch.full((2,), T + 1 + off, device="cuda"))
+            out.append(gd.step(cur).clone())
+            runs.append(out)
+    finally:
+        m.rope_cos, m.rope_sin = cos, sin
+    for a, b in zip(*runs):
+        assert torch.equal(a, b)
