@@ -144,7 +144,8 @@ class _Workspace(dict):
     """The buffers of one forward pass by name: made at their first use and
     used again by every later layer of the pass (launches of one pass run in
     order on one stream, so a buffer's readers are ahead of its next writer).
-    A pass makes its own, so concurrent passes share nothing."""
+    A pass makes its own, so concurrent passes share nothing, and drops them
+    before the LM head. A layer that needs another shape gets a new buffer."""
 
     def __init__(self, device):
         super().__init__()
@@ -153,7 +154,7 @@ class _Workspace(dict):
 
     def buf(self, name, shape, dtype):
         t = self.get(name)
-        if t is None:
+        if t is None or t.shape != shape or t.dtype != dtype:
             t = self[name] = torch.empty(shape, dtype=dtype, device=self.device)
         return t
 
@@ -399,6 +400,7 @@ class IntQwen3:
             for li, L in enumerate(self.layers):
                 nxt = self.layers[li + 1] if li + 1 < self.n_layers else None
                 self._layer(ws, L, nxt, B, T, h, k_res, x8, xm, xk, pos, cache, S_past, S, static)
+        ws.clear()
         if not static:
             cache.length = S
         if head_rows is not None:
@@ -509,7 +511,7 @@ class IntQwen3:
         if plan is not None:
             # long rows: Q/K/V epilogue, then the split-S attention
             chunk, nsp = plan
-            q8 = ws.buf("q8", (B, nq, 1, hd), torch.int8)
+            q8 = ws.buf("q8", (B, nq * hd), torch.int8)
             tpos = ws.buf("tpos", (B, nq, 1), I64)
             call("detllm_qkv_epilogue", P, ns, st, B, 1, nq, nkv, xm, xk, pos,
                  *L.epi, self.rope_cos, self.rope_sin, self.max_pos, q8, tpos, None,
@@ -621,7 +623,7 @@ class IntQwen3:
     def _attention(self, ws: _Workspace, L, B, T, P, ns, st, xm, xk, pos, cache, S_past, S, static,
                    attn):
         nq, nkv, hd, li = self.n_q, self.n_kv, self.hd, L.idx
-        q8 = ws.buf("q8", (B, nq, T, hd), torch.int8)
+        q8 = ws.buf("q8", (B * T, nq * hd), torch.int8)
         tpos = ws.buf("tpos", (B, nq, T), I64)
         call("detllm_qkv_epilogue", P, ns, st, B, T, nq, nkv, xm, xk, pos,
              *L.epi, self.rope_cos, self.rope_sin, self.max_pos, q8, tpos, None,
@@ -689,7 +691,9 @@ class IntQwen3:
     def _after_attention(self, ws: _Workspace, L, nxt, B, T, attn, h, k_res, x8, xm, xk):
         """attn: (context partials, nsplit, split_stride) as _attend returns."""
         R, H, nq, hd, I_ = B * T, self.hidden, self.n_q, self.hd, self.inter
-        a8 = ws.buf("a8", (R, nq * hd), torch.int8)
+        # (prefill: the layer's footprint matters; the queries are read, and the
+        # o product is, before what takes their buffers here is written)
+        a8 = ws.buf("q8", (R, nq * hd), torch.int8)
         am, ak, ym, yk = (ws.buf(n, (R,), I64) for n in ("am", "ak", "ym", "yk"))
         # decode sizes: the merge and the SwiGLU leave their scale fits to the
         # residual kernel after the next GEMM (same integers)
@@ -710,7 +714,7 @@ class IntQwen3:
         call("detllm_swiglu_quant", P, ns, st, R, I_, xm, xk, L.gate_m, L.gate_k, L.up_m,
              L.up_k, L.ds_m, L.ds_k, y8, ym, yk, *self._next_gemm(L.wd, R), dfit)
         P, ns, st = self._gemm(y8, L.wd, (L.down_m,) if nxt is None else (L.down_m, nxt.as_m),
-                               ws=ws, name="P_d")
+                               ws=ws, name="P_o" if R > 64 else "P_d")
         sm_m, sm_k = (nxt.as_m, nxt.as_k) if nxt is not None else (None, 0)
         call("detllm_residual_normq", P, ns, st, R, H, ym, yk, L.down_m, L.down_k, 20, h, k_res,
              sm_m, sm_k, x8, xm, xk, *self._next_gemm(None if nxt is None else nxt.wqkv, R), dfit)
