@@ -95,10 +95,17 @@ def _missing(path):
 
 
 def native():
-    """The native binding module (raises LibraryMissing when it is not built)."""
-    if not os.path.exists(NATIVE_PATH):
-        raise _missing(NATIVE_PATH)
-    return importlib.import_module(__package__ + "._native")
+    """The native binding module (raises LibraryMissing when it is not built,
+    or does not load: built for another torch, or its library is missing)."""
+    for path in (NATIVE_PATH, LIB_PATH):
+        if not os.path.exists(path):
+            raise _missing(path)
+    importlib.invalidate_caches()      # it may have been built since a first try
+    try:
+        return importlib.import_module(__package__ + "._native")
+    except ImportError as e:
+        raise LibraryMissing(f"{NATIVE_PATH} does not load ({e}); build it again: `python -c "
+                             "'import __graft_entry__ as g; g.build()'`") from e
 
 
 def load():
@@ -116,11 +123,6 @@ def load():
     _entries.update(native().entries())
     _lib = lib
     return lib
-
-
-def stream_handle(stream=None) -> int:
-    s = stream if stream is not None else torch.cuda.current_stream()
-    return s.cuda_stream
 
 
 def gemv_plan(M: int, N: int, K: int) -> int:

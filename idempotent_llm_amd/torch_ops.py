@@ -21,7 +21,7 @@ validity mask).
 
 from __future__ import annotations
 
-import os
+import threading
 
 import torch
 
@@ -169,9 +169,39 @@ def attn_decode(q8, tpos, kpool, vpool, table, valid, S, err):
     return q8.new_empty(q8.shape[0], q8.shape[1] * 128, dtype=I64)
 
 
-if os.path.exists(_lib.NATIVE_PATH):
-    _lib.native()      # registers the kernels
-else:
-    # no kernels: every call raises LibraryMissing, as the other entries do
-    for _name in OPS:
-        torch.library.impl(f"{NS}::{_name}", "CUDA")(lambda *a, **k: _lib.native())
+# Loading the native binding registers the kernels. Where it cannot be loaded
+# (not built, or built for another torch), the import goes on and a call of an
+# operator raises, as the other entries do; a call after it has been built
+# loads it.
+_stand_ins = None
+_loading = threading.Lock()
+
+
+def _load_kernels():
+    global _stand_ins
+    with _loading:
+        if _stand_ins is None:
+            return
+        _stand_ins._destroy()     # (before the kernels of the same key are registered)
+        try:
+            _lib.native()
+        except Exception:
+            _register_stand_ins()
+            raise
+        _stand_ins = None
+
+
+def _register_stand_ins():
+    global _stand_ins
+    _stand_ins = torch.library.Library(NS, "IMPL")
+    for name in OPS:
+        def call_again(keyset, *args, _op=getattr(torch.ops.detllm_rocm, name).default, **kwargs):
+            _load_kernels()
+            return _op.redispatch(keyset, *args, **kwargs)
+        _stand_ins.impl(name, call_again, "CUDA", with_keyset=True)
+
+
+try:
+    _lib.native()
+except _lib.LibraryMissing:
+    _register_stand_ins()
