@@ -184,8 +184,9 @@ __global__ __launch_bounds__(256, 2) void k_attn_prefill(PrefillArgs a) {
     }
   };
   // A block of few pages keeps all of K and V in the ring for its three
-  // passes: one memory round trip, beside the mask's, and no barrier per tile
-  // (a round trip of each pass's loads is most of a short prompt's launch).
+  // passes: its loads are made once, before the mask's, with no barrier per
+  // tile (a round trip of each pass's loads is most of a short prompt's
+  // launch). The second page's id is waited for behind the first page's loads.
   const bool resident = ntiles2 <= PF_RESIDENT;
   if (resident) {
     for (int i = 0; i < ntiles2; ++i)
@@ -203,7 +204,7 @@ __global__ __launch_bounds__(256, 2) void k_attn_prefill(PrefillArgs a) {
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
       const int s = (i0 + 4 * u) * 64 + lane;
-      const uint32_t v = vrow[s < a.S ? s : 0];  // unconditional: one wait for all four
+      const uint32_t v = vrow[s < a.S ? s : 0];  // (the guard below still waits for each)
       f[u] = (i0 + 4 * u < ntiles && s < a.S) ? v : 0u;
     }
 #pragma unroll
@@ -1279,7 +1280,8 @@ __global__ __launch_bounds__(256) void k_attn_split_pv(SplitArgs sa) {
   const int lo = c * sa.chunk;
   const i64 q0 = (i64)b * a.n_q + kvh * G;
   int64_t* outp = a.out + (sa.add ? 0 : c * sa.out_stride) + q0 * 128;
-  // (the pages, constants and maxima load beside the device's slot count)
+  // (none of these depends on the device's slot count, which loads last: the
+  // page id, then per head the constant and its chunk maxima, each waited for)
   const int npg = (::min(sa.chunk, a.S - lo) + DI_PAGE - 1) / DI_PAGE;
   const int pgv = tid < npg ? a.kv.page(b, (i64)lo + (i64)tid * DI_PAGE) : -1;
   i64 tph[G], hmax[G];

@@ -77,8 +77,8 @@ bool convert(PyObject* o, T* out) {
 // Runs entry f on `args` (every parameter but a trailing stream, which is
 // `stream`): the entry's return code, or -1 with a Python exception set.
 template <class... A, size_t... I>
-bool run(int (*f)(A...), PyObject* const* args, hipStream_t stream, bool has_stream,
-         std::index_sequence<I...>, int* rc) {
+bool run(int (*f)(A...), PyObject* const* args, hipStream_t stream, std::index_sequence<I...>,
+         int* rc) {
   std::tuple<A...> v;
   constexpr size_t N = sizeof...(A);
   auto one = [&](auto idx) {
@@ -92,7 +92,6 @@ bool run(int (*f)(A...), PyObject* const* args, hipStream_t stream, bool has_str
     }
   };
   if (!(one(std::integral_constant<size_t, I>{}) && ...)) return false;
-  (void)has_stream;
   Py_BEGIN_ALLOW_THREADS
   *rc = f(std::get<I>(v)...);
   Py_END_ALLOW_THREADS
@@ -113,7 +112,7 @@ struct Bind<F> {
   static constexpr bool has_stream =
       std::is_same_v<std::tuple_element_t<sizeof...(A) - 1, std::tuple<A...>>, hipStream_t>;
   static bool call(PyObject* const* args, hipStream_t s, int* rc) {
-    return run(F, args, s, has_stream, std::index_sequence_for<A...>{}, rc);
+    return run(F, args, s, std::index_sequence_for<A...>{}, rc);
   }
   static constexpr Entry entry(const char* name) {
     return Entry{name, (int)sizeof...(A) - (has_stream ? 1 : 0), has_stream, &call};

@@ -808,3 +808,17 @@ def test_norm_quant_every_path(C, big_sm):
     xk = torch.empty(R, dtype=torch.int64, device="cuda")
     call("detllm_norm_quant", g(h), R, C, g(sm_m), 15, x8, xm, xk)
     eq(x8, want[0]); eq(xm, want[1][:, 0]); eq(xk, want[2][:, 0])
+
+
+@pytest.mark.parametrize("shape", [(1, 1), (5, 3), (64, 64), (63, 65), (129, 200), (3, 17, 31),
+                                   (2, 3, 70, 66), (4, 1, 100)])
+def test_transpose_i8(shape):
+    """detllm_transpose_i8 (backends.transpose_i8) on ragged tiles, batches,
+    and a non-contiguous operand."""
+    from idempotent_llm_amd.backends import transpose_i8
+    print(f"[transpose_i8 {shape}]", flush=True)
+    x = torch.randint(-128, 128, shape, dtype=torch.int8, device="cuda")
+    assert torch.equal(transpose_i8(x), x.transpose(-1, -2))
+    y = torch.randint(-128, 128, (*shape[:-1], shape[-1] + 3), dtype=torch.int8,
+                      device="cuda")[..., 1:shape[-1] + 1]
+    assert torch.equal(transpose_i8(y), y.transpose(-1, -2))
