@@ -145,14 +145,16 @@ struct HeadRed {
 // A mantissa operand of qk_head_f64 as an exact double, and whether it lies
 // inside the bound that needs (a float, which holds any integer below 2^24,
 // was checked when it was made: it takes half a double's registers).
-constexpr i64 QKV_WM_LIM = (i64)1 << 21, QKV_G_LIM = (i64)1 << 12, QKV_QS_LIM = (i64)1 << 15;
+// (The quantiser's widest: 16, 14 and 14 bits.)
+constexpr i64 QKV_WM_LIM = (i64)1 << 21, QKV_G_LIM = (i64)1 << 14, QKV_QS_LIM = (i64)1 << 15;
+constexpr double QKV_R_LIM = 0x1p38;  // rotated values (qk_head_f64)
 __device__ __forceinline__ double mant_f64(i64 x) { return (double)(int32_t)x; }
 __device__ __forceinline__ double mant_f64(float x) { return (double)x; }
 __device__ __forceinline__ bool mant_ok(i64 x, i64 lim) { return in_range(x, lim); }
 __device__ __forceinline__ bool mant_ok(float, i64) { return true; }
 
 // requant_i8_static(kk, 1, k_rowk, 1, 0, kq_m, kq_k) of one rotated K value
-// (an exact double below 2^52): n = r << up, rhad(n, den) clamped
+// (an exact double below 2^38): n = r << up, rhad(n, den) clamped
 __device__ __forceinline__ int kq_quant(double r, const KqChan& q) {
   const double n = ldexp(r, (int)imin(q.up, 64));
   const i64 lim = (i64)1 << 49;  // 2 |n| + den < 2^51 for the estimate
@@ -175,10 +177,14 @@ __device__ __forceinline__ int kq_quant(double r, const KqChan& q) {
 //  * rms = isqrt(mean) >= 2^21 unless the head is zero (the largest |y 2^u|
 //    is at least 2^25), so the normalised values rhad(y 2^u 2^20, rms) are
 //    below 11.32 * 2^20 < 2^24 in magnitude (|y 2^u| <= sqrt(128 mean + 64)),
-//    and with |gamma_m| < 2^12 the gamma products a stay below 2^36;
-//  * the RoPE sums a cos + a' sin (int16 tables, |entry| <= 2^15) are exact
-//    doubles below 2^52, the rotated values r = rshift_round(., 14) below
-//    2^38, and with |qs_m| < 2^15 the smoothed q = r qs_m below 2^53.
+//    and with |gamma_m| < 2^14 the gamma products a stay below 2^37.6;
+//  * a RoPE sum a cos + a' sin (int16 tables, |entry| <= 2^15) is one fma of
+//    an exact product (below 2^53): exact if it is below 2^52, and 2^52 or
+//    more if the sum is. Then r = rshift_round(., 14) reaches 2^38, and that is
+//    checked (Q: through the head's maximum; K: by kquant). Tables of cosines
+//    and sines at 14 bits never come there: a^2 + a'^2 < (11.32 2^34)^2, so
+//    their sums stay below 2^51.6;
+//  * with |r| < 2^38 and |qs_m| < 2^15 the smoothed q = r qs_m is below 2^53.
 // The Q quotients rhad(127 |q|, am) come from fp64 estimates for every am
 // below 2^53 (exact below 2^43 as in quant_row; above, checked per element).
 // Returns false (uniform over the head's lanes) for a head outside them, or
@@ -187,7 +193,8 @@ __device__ __forceinline__ int kq_quant(double r, const KqChan& q) {
 // max(max |q|, 1). W: int64 mantissas, checked here, or floats that the
 // caller checked (ok0) and made once for several rows.
 // kquant(r, o): the K head's int8 values from its rotated ones (false: it
-// could not, and the head takes the integer routines).
+// could not, or some |r| reaches 2^38, and the head takes the integer
+// routines).
 template <int N, bool WAVE, class W, class KqF>
 __device__ __forceinline__ bool qk_head_f64(bool is_q, const int32_t (&p)[N],
                                             const W (&wm)[N], const W (&gm)[N],
@@ -242,13 +249,15 @@ __device__ __forceinline__ bool qk_head_f64(bool is_q, const int32_t (&p)[N],
   }
   // QK smoothing, then quant_i8_pertoken's quotients (quant_row's two forms)
   double q[N];
-  double g = 0.0;
+  double g = 0.0, rm = 0.0;
 #pragma unroll
   for (int i = 0; i < N; ++i) {
     q[i] = r[i] * mant_f64(qs[i]);
     g = fmax(g, fabs(q[i]));
+    rm = fmax(rm, fabs(r[i]));
   }
-  const double amu = f64_from_bits(red.max(f64_bits(g)));
+  const double amu = f64_from_bits(red.max(f64_bits(rm < QKV_R_LIM ? g : 0x1p53)));
+  if (DI_UNLIKELY(amu >= 0x1p53)) return false;
   const i64 am = imax((i64)amu, 1);
   const DivEst Dq = make_divest(am, 127.0);
   *am_out = am;
@@ -514,7 +523,7 @@ __device__ __forceinline__ void qkv_head_compute(const QKVArgs& a, int r, int sl
                                 [&](const double (&rv)[2], int (&ov)[2]) {
 #pragma unroll
                                   for (int i = 0; i < 2; ++i) ov[i] = kq_quant(rv[i], kq(i));
-                                  return true;
+                                  return __ballot(!(fmax(fabs(rv[0]), fabs(rv[1])) < QKV_R_LIM)) == 0;
                                 },
                                 o, &am);
   }
@@ -785,7 +794,7 @@ __device__ __forceinline__ uint32_t qkv_rows_kind(const QKVArgs& a, int R, int r
   // below is fma(|r|, 2^up r, k), an exact scaling)
   float gm[8], qs[8];
   double qa[8], kb[8];
-  double klim = 0.0;  // |r| below which every channel's divisor estimate holds
+  double klim = 0.0;  // |r| below which r is exact and every channel's divisor estimate holds
   {
     i64 w[8];
     load8(gam, w);
@@ -818,7 +827,7 @@ __device__ __forceinline__ uint32_t qkv_rows_kind(const QKVArgs& a, int R, int r
       qs[i] = (float)(int32_t)w[i];
     }
   } else {
-    klim = 0x1p49;
+    klim = QKV_R_LIM;
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
       const KqChan q = kq(i);

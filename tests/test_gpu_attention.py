@@ -521,8 +521,19 @@ def _plant(prm, variant, nq, nkv):
         prm.update(q_m=q_m, k_m=k_m, v_m=v_m, qs_m=qs_m, kq_m=kq_m, kq_k=kq_k)
     elif variant == "gamma":
         g = cl("q_norm_m")
-        g[9] = 1 << 12                          # every Q head: gamma beyond the doubles
+        g[9] = 1 << 14                          # every Q head: gamma beyond the doubles
         prm["q_norm_m"] = g
+    elif variant in ("gamma14", "tables"):      # the quantiser's 14-bit gammas, up to the limit
+        for k in ("q_norm_m", "k_norm_m"):
+            g = cl(k) * 4
+            g[::3] *= -1
+            g[3], g[67], g[9] = (1 << 14) - 1, -((1 << 14) - 1), (1 << 14) - 1
+            prm[k] = g
+        if variant == "tables":                 # entries of any size at half of the positions
+            for k, v in (("cos", 32767), ("sin", -32768)):
+                t = cl(k)
+                t[::2] = v
+                prm[k] = t
     return prm
 
 
@@ -620,6 +631,13 @@ def _rows_per_lane(variant, B, T, slot):
                       dtype=torch.int32)
     P[0, 5, 9 * hd:10 * hd] = 0
     P[0, R - 1, (nq + 6) * hd:(nq + 7) * hd] = 0
+    if variant == "tables":     # heads of one RoPE pair: rotated sums from 2^52 on
+        heads = P.view(R, nq + 2 * nkv, hd)
+        for r in (0, 2, 3, R // 2, R - 2):
+            for h in (1, 7, nq - 1, nq, nq + 3):
+                keep = heads[r, h, [3, 67]].abs() + (1 << 18)
+                heads[r, h] = 0
+                heads[r, h, 3], heads[r, h, 67] = keep[0], keep[1]
     P = P.cuda()
     xm = torch.randint(1 << 15, 1 << 16, (R,), generator=rnd, dtype=I64)
     xm[R // 2] = (1 << 40) + 7
@@ -811,4 +829,14 @@ def test_qkv_epilogue_rows_per_lane_lines(variant, B, T, slot):
     """The same on both sides of the line to four rows per lane (49152 (row,
     head) pairs: 1536 rows of 32 heads) and on the line to two (21504: 672
     rows); the sizes above take two."""
+    _rows_per_lane(variant, B, T, slot)
+
+
+@pytest.mark.parametrize("variant", ["gamma14", "tables"])
+@pytest.mark.parametrize("B,T,slot", [(7, 1, 50), (1, 100, 3), (3, 224, 1), (1, 1536, 126)])
+def test_qkv_epilogue_wide_gamma(variant, B, T, slot):
+    """Gammas at the quantiser's 14 bits (fit_gamma_dyadic) keep the fp64
+    forms, in the one-token layout and with one, two and four rows per lane;
+    with tables of any int16 entries the rotated sums of some heads pass 2^52
+    and those heads take the integer routines."""
     _rows_per_lane(variant, B, T, slot)
