@@ -630,8 +630,8 @@ namespace di {
 // lane's NG consecutive slots of V go out as one word instead of NG bytes.
 // Measured at 2048 rows of 32 heads (32 MB of product), one row against four
 // rows per lane: launched back to back 34.8 -> 25.0 us (in a prefill's trace,
-// its inputs fresh from the product, 29), vector instructions 14.3 M -> 11.0 M
-// (70 % of the issue slots), 4096 rows 63 -> 43 us. The kinds are separate code
+// its inputs fresh from the product, 30), vector instructions 14.3 M -> 10.6 M
+// (17 us of issue time), 4096 rows 63 -> 43 us. The kinds are separate code
 // (qkv_rows_kind), and rows outside the fp64 forms' bounds are redone after the
 // passes: either one inside the passes costs enough registers to halve the
 // waves in flight. Four waves per SIMD still take spills at NG = 4 (68 vector

@@ -50,7 +50,8 @@ GREEDY_CHUNK = 2048
 # slots the decode attention scans at most (int32 MFMA accumulators of P.V:
 # 128 * 128 * S < 2^31)
 DEC_MAX_SLOTS = 131071
-# decode rows scanning at least this many slots use the split-S attention
+# decode rows scanning at least this many slots are cut as detllm_attn_split_plan
+# says (in one chunk: the one-block kernel)
 SPLIT_MIN_SLOTS = 2048
 # decode batches up to this many rows have the attention write the merge's
 # row statistics: one row takes the o-GEMV that quantises its own K range of
