@@ -1617,16 +1617,20 @@ int detllm_qkv_attn_decode_ext(const int32_t* P, int nsplit, int64_t split_strid
 // 36.8 / 33.8 / 42.1.
 //
 // From 256 pairs on the pairs fill the chip by themselves, and scores and
-// partials through HBM only cost: as few chunks as the limits allow, of even
-// length, and where that is one (4096 slots at 1 or 2 query heads per kv head)
-// the one-block kernel takes the row. us per decode step of 4 layers, 16 / 8
+// partials through HBM only cost: where one chunk holds the row (4096 slots at
+// 1 or 2 query heads per kv head) the one-block kernel takes it, and longer
+// rows are cut evenly, into as few chunks as the limits allow from 512 pairs
+// on, below at 2048 slots (two chunks of 4096 leave a chip of 256 to 511 blocks
+// half idle when the second is short). us per decode step of 4 layers, 16 / 8
 // heads, one block / chunks of 1024 / 2048 / 4096: 32 x 4000 460 / 509 / 518 /
-// -, 64 x 4000 672 / 788 / 754 / -, 128 x 4000 1135 / 1305 / 1267 / -, 32 x
-// 8100 855 / 783 / 726 / 741, 64 x 8100 1376 / 1287 / 1207 / 1176, 128 x 8100
-// 2549 / 2302 / 2188 / 2140 (24 rows, 192 pairs: 4000 431 / 457 / 493 / -,
-// 8100 819 / 666 / 625 / 692). us per call, 32 / 8 heads, one block / 1024 /
-// 2048: 64 x 4096 160 / 148 / 135, 128 x 4096 336 / 279 / 263; at 2048 slots
-// one block against two chunks 37 / 39 (32 rows), 47 / 63 (64), 100 / 135 (128).
+// -, 64 x 4000 672 / 788 / 754 / -, 128 x 4000 1135 / 1305 / 1267 / -; in a
+// launch sized for 8192 slots 32 x 4200 569 / 547 / 539 / 572, 32 x 8100 855 /
+// 783 / 726 / 741, 48 x 5000 888 / 784 / 750 / 797, 64 x 4200 851 / 840 / 813 /
+// 811, 64 x 8100 1376 / 1287 / 1207 / 1176, 128 x 8100 2549 / 2302 / 2188 / 2140
+// (24 rows, 192 pairs: 4000 431 / 457 / 493 / -, 8100 819 / 666 / 625 / 692). us
+// per call, 32 / 8 heads, one block / 1024 / 2048: 64 x 4096 160 / 148 / 135,
+// 128 x 4096 336 / 279 / 263; at 2048 slots one block against two chunks 37 / 39
+// (32 rows), 47 / 63 (64), 100 / 135 (128).
 int detllm_attn_split_plan(int B, int S, int n_q, int n_kv, int* chunk, int* nsplit) {
   if (!chunk || !nsplit || B <= 0 || S <= 0 || n_q <= 0 || n_kv <= 0 || n_q % n_kv) return DI_EINVAL;
   const int G = n_q / n_kv;
@@ -1635,7 +1639,8 @@ int detllm_attn_split_plan(int B, int S, int n_q, int n_kv, int* chunk, int* nsp
   const i64 blocks = (i64)B * n_kv;
   i64 ch;
   if (blocks >= 256) {
-    const i64 ns = ((i64)S + cmax - 1) / cmax;
+    const i64 longest = S <= cmax || blocks >= 512 ? cmax : imin(cmax, 2048);
+    const i64 ns = ((i64)S + longest - 1) / longest;
     ch = ((i64)S + ns - 1) / ns;
   } else {
     const i64 want = (256 + blocks - 1) / blocks;

@@ -370,8 +370,9 @@ int detllm_attn_decode_split_sum(const int8_t* q8, const int64_t* tpos, const in
 
 /* The chunking detllm_attn_decode_split is tuned for at (B, S, n_q, n_kv).
  * Below 256 (row, kv head) pairs about 256 blocks: chunks of 256 to 1024 slots,
- * at most 16 per row where the longest chunk allows it; from 256 pairs on as
- * few chunks as it allows. The longest chunk is 4096 slots, less above 2 query
+ * at most 16 per row where the longest chunk allows it; from 256 pairs on one
+ * chunk where it allows it, else even ones of at most 2048 slots (from 512
+ * pairs on the longest). The longest chunk is 4096 slots, less above 2 query
  * heads per kv head (3072 at 4, 1536 at 8). *nsplit of 1: detllm_attn_decode
  * (or detllm_qkv_attn_decode) is the faster call. Writes *chunk, *nsplit. */
 int detllm_attn_split_plan(int B, int S, int n_q, int n_kv, int* chunk, int* nsplit);

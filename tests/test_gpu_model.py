@@ -383,7 +383,7 @@ def test_logits_digest_matches_host_formula(case):
 
 def test_split_attention_of_many_rows(case, monkeypatch):
     """One decode step of 128 rows (256 (row, kv head) pairs) past the longest
-    chunk: through the split-S attention in two chunks, and through the
+    chunk: through the split-S attention in three chunks, and through the
     one-block kernel, the same logits; one slot less than the longest chunk
     stays whole."""
     rec, m, _ = case
@@ -397,7 +397,7 @@ def test_split_attention_of_many_rows(case, monkeypatch):
     pos = (torch.arange(n + 1, device="cuda") % 1000).expand(B, n + 1)
     valid = torch.rand(B, n + 1, device="cuda", generator=g) < 0.9
     valid[:, n] = True
-    assert m._split_plan(B, 4096) is None and m._split_plan(B, n + 1)[1] == 2
+    assert m._split_plan(B, 4096) is None and m._split_plan(B, n + 1)[1] == 3
     cache, runs = KVCache(), []
     rows = torch.zeros(B, dtype=I64, device="cuda")
     for lo in range(0, n, step):

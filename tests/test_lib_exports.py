@@ -137,9 +137,9 @@ def test_missing_library_fails_loudly(monkeypatch, tmp_path):
 @pytest.mark.parametrize("n_q,n_kv", [(8, 8), (16, 8), (32, 8), (64, 8), (8, 1), (4, 2)])
 def test_attn_split_plan_host_entry(n_q, n_kv):
     """Every plan is one the split launch takes, of chunks that cover the
-    slots. From 256 (row, kv head) pairs on a row is cut no further than the
-    longest chunk makes necessary: rows within it stay whole (the one-block
-    kernel), longer ones are cut evenly."""
+    slots. From 256 (row, kv head) pairs on rows within the longest chunk stay
+    whole (the one-block kernel) and longer ones are cut evenly, no further
+    than that chunk (2048 slots below 512 pairs) makes necessary."""
     from idempotent_llm_amd._lib import attn_split_plan
     G = n_q // n_kv
     longest = min(48 * 1024 // (4 * G) // 128 * 128, 4096)
@@ -150,5 +150,6 @@ def test_attn_split_plan_host_entry(n_q, n_kv):
             assert chunk % 128 == 0 and 256 <= chunk <= longest, (B, S, chunk)
             assert ns == -(-S // chunk), (B, S, chunk, ns)
             if B * n_kv >= 256:
-                assert ns == -(-S // longest), (B, S, chunk, ns)
+                most = longest if S <= longest or B * n_kv >= 512 else min(longest, 2048)
+                assert ns == -(-S // most), (B, S, chunk, ns)
                 assert ns == 1 or chunk - S / ns < 128, (B, S, chunk, ns)
